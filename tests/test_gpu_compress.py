@@ -525,6 +525,43 @@ def test_compress_paged_values_appends(dev, bits):
     sel = rows[:, :, :][written[:, None, :].repeat(H, 1)]
     assert np.array_equal(pl_got2["idx"][sel], pl_want["idx"][sel])
 
+# Token runs (first slot, tokens; first slot None: that many tokens skipped with slot -3, -2, ...)
+# whose ends fall everywhere in a chunk of 4 slots, in a wave's 16 rows and in a workgroup's 64.
+_RUNS = {
+    "single": [(7, 1)],
+    "short": [(5, 2), (33, 3), (50, 1), (19, 1)],
+    "wave_edges": [(1, 16), (34, 15), (67, 17), (98, 14)],
+    "skipped": [(2, 5), (None, 3), (18, 19), (None, 2), (48, 7)],
+    "two_passes": [(13, 3), (17, 19), (39, 4), (46, 33), (81, 47)],
+    "long": [(3, 61), (66, 70), (140, 130), (273, 200)],
+}
+
+
+@pytest.mark.parametrize("runs", list(_RUNS))
+@pytest.mark.parametrize("bits,dtype,idt", [(2, torch.bfloat16, torch.int32), (3, torch.float16, torch.int64),
+                                            (4, torch.bfloat16, torch.int64), (3, torch.float32, torch.int32)])
+def test_compress_paged_values_ragged_runs(dev, runs, bits, dtype, idt):
+    """One call over runs that start and end off a multiple of 4 slots writes the bytes of one call per
+    token (whose rows set their own fields with atomics), over a cache that held other data."""
+    from turboquant.kernels.paged import PagedKVFormat, allocate_cache, compress_paged
+    slots, neg = [], -3
+    for first, n in _RUNS[runs]:
+        slots += list(range(first, first + n)) if first is not None else list(range(neg, neg + n))
+    T, H, bs, nb = len(slots), 3, 16, 32
+    g = torch.Generator().manual_seed(bits)
+    x = torch.randn(T, H, 128, generator=g).to(dtype).to(dev)
+    sl = torch.tensor(slots, dtype=idt, device=dev)
+    fmt = PagedKVFormat(bits=bits, qjl=False, block_size=bs, layout="values")
+    cb = tuple(t.to(dev) for t in _codebook(bits))
+    got = allocate_cache(nb, H, fmt, device=dev)
+    got.random_(0, 256, generator=torch.Generator(device=dev).manual_seed(1))
+    want = got.clone()
+    compress_paged(x, sl, got, fmt, *cb)
+    for t in range(T):
+        compress_paged(x[t:t + 1], sl[t:t + 1], want, fmt, *cb)
+    assert torch.equal(got, want)
+
+
 
 def test_compress_paged_kv_rejections(dev):
     from turboquant.kernels.paged import PagedKVFormat, allocate_cache, compress_paged_kv

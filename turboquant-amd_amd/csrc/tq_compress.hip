@@ -483,30 +483,22 @@ __device__ __forceinline__ void shl_words(const uint32_t (&a)[BITS], uint32_t s,
     }
 }
 
-// Writes this lane's fields into the values layout.  Rows 4a..4a+3 of a workgroup that land on
-// slots 4k..4k+3 fill whole chunks: their slices are exchanged through this group's part of
-// xchg and each lane stores one chunk.  Any other row sets its own fields with atomic and / or on
+// Writes this lane's fields into the values layout.  Four consecutive rows of the wave that land on
+// slots 4k..4k+3 (full: the lane's row is one of them) fill whole chunks, wherever in the wave they
+// start: their slices are exchanged through part gi of the wave's xchg (gi counts the wave's full
+// groups) and each lane stores one chunk.  Any other row sets its own fields with atomic and / or on
 // the chunk words (other rows of the chunk, written by other launches or workgroups, are
-// untouched).  Lane layouts: 4 consecutive lanes per row (a group of 4 rows is lanes
-// 16a'..16a'+15 of one wave, slice i of lane q is chunk 4q + i), or GROUPS, the matrix-core
-// rows (row l & 15, lane group q = l >> 4: a group of 4 rows is lanes 4a' + {0..3} + 16 {0..3},
-// slice i of lane q is chunk 4i + q).
+// untouched).  Slice i of lane q is chunk 4q + i with 4 consecutive lanes per row, chunk 4i + q in
+// GROUPS, the matrix-core rows (row l & 15, lane group q = l >> 4).
 template <int BITS, bool GROUPS>
-__device__ __forceinline__ void store_values(const ValueSlices<BITS>& vs, bool write, int64_t slot, uint8_t* tile,
-                                             int64_t r_in_blk, int q, uint32_t* xchg) {
+__device__ __forceinline__ void store_values(const ValueSlices<BITS>& vs, bool write, bool full, int gi, int r16, int rows,
+                                             uint32_t plink, uint8_t* tile, int64_t r_in_blk, int q, uint32_t* xchg) {
     constexpr int VS = BITS == 3 ? 4 : BITS;  // words per slice in the exchange (b64 / b128 access)
-    const int lane = threadIdx.x & 63;
-    const int rr = GROUPS ? (lane & 3) : ((threadIdx.x >> 2) & 3);  // row of the lane within its group of 4 rows
-    const int64_t s0 = __shfl(slot, GROUPS ? (lane & 12) : (lane & ~12));
-    const bool ok = write && (s0 & 3) == 0 && slot == s0 + rr;
-    const uint64_t bal = __builtin_amdgcn_ballot_w64(ok);
-    const bool full = GROUPS ? ((bal >> (lane & 12)) & 0x000F000F000F000Full) == 0x000F000F000F000Full
-                             : ((bal >> (lane & 48)) & 0xffffull) == 0xffffull;
+    const int rr = (int)(r_in_blk & 3);       // row of the lane within its group of 4 rows
     uint8_t* sub = tile + (r_in_blk & ~(int64_t)15) * (16 * BITS);
     const int g = (int)((r_in_blk & 15) >> 2);
     if (full) {
-        const int grp = GROUPS ? ((threadIdx.x >> 6) * 4 + ((lane & 15) >> 2)) : (threadIdx.x >> 4);
-        uint32_t* gx = xchg + grp * (64 * VS);  // this group: [chunk][row][VS]
+        uint32_t* gx = xchg + ((threadIdx.x >> 6) * 4 + gi) * (64 * VS);  // this group: [chunk][row][VS]
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             uint32_t* d = gx + ((GROUPS ? 4 * i + q : q * 4 + i) * 4 + rr) * VS;
@@ -543,29 +535,55 @@ __device__ __forceinline__ void store_values(const ValueSlices<BITS>& vs, bool w
         uint32_t* ch = reinterpret_cast<uint32_t*>(sub + (16 * g + 4 * q + rr) * (4 * BITS));
 #pragma unroll
         for (int k = 0; k < BITS; ++k) ch[k] = out[k];
-    } else if (write) {
-        const uint32_t sh = (uint32_t)(BITS * (r_in_blk & 3));
-        uint32_t m0[BITS];
+    }
+    if (__builtin_amdgcn_ballot_w64(write && !full)) {
+        // chunks of which the wave holds 1-3 rows: the chunk's first row here sets the fields of all
+        // of them, one and / or pair per word (the pairs of one word follow each other at the memory
+        // side, so one pair per row made every end of a run wait for up to eight)
+        const bool ends = write && !full && (r16 == 0 || !((plink >> r16) & 1u));
+        const int n1 = (int)((plink >> (r16 + 1)) & 7u);  // rows r16 + 1 .. + 3 continue their predecessors
+        const int left = rows - 1 - r16;
+        const int n = (n1 & 1) && left >= 1 ? ((n1 & 2) && left >= 2 ? ((n1 & 4) && left >= 3 ? 3 : 2) : 1) : 0;
+        uint32_t m0[BITS], m[BITS];
 #pragma unroll
         for (int k = 0; k < BITS; ++k) m0[k] = value_field_mask<BITS>(k);
-        uint32_t m[BITS];
-        shl_words<BITS>(m0, sh, m);
+        shl_words<BITS>(m0, (uint32_t)(BITS * rr), m);
+#pragma unroll
+        for (int d = 1; d < 4; ++d) {
+            uint32_t ms[BITS];
+            shl_words<BITS>(m0, (uint32_t)(BITS * ((rr + d) & 3)), ms);
+#pragma unroll
+            for (int k = 0; k < BITS; ++k) m[k] |= d <= n ? ms[k] : 0u;
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             uint32_t b[BITS];
-            shl_words<BITS>(vs.w[i], sh, b);
-            uint32_t* ch = reinterpret_cast<uint32_t*>(sub + (16 * g + (GROUPS ? 4 * i + q : 4 * q + i)) * (4 * BITS));
+            shl_words<BITS>(vs.w[i], (uint32_t)(BITS * rr), b);
 #pragma unroll
-            for (int k = 0; k < BITS; ++k) {
-                __hip_atomic_fetch_and(ch + k, ~m[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_fetch_or(ch + k, b[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int d = 1; d < 4; ++d) {
+                uint32_t o[BITS], os[BITS];
+#pragma unroll
+                for (int k = 0; k < BITS; ++k) o[k] = __shfl_down(vs.w[i][k], GROUPS ? d : 4 * d);
+                shl_words<BITS>(o, (uint32_t)(BITS * ((rr + d) & 3)), os);
+#pragma unroll
+                for (int k = 0; k < BITS; ++k) b[k] |= d <= n ? os[k] : 0u;
+            }
+            if (ends) {
+                uint32_t* ch = reinterpret_cast<uint32_t*>(sub + (16 * g + (GROUPS ? 4 * i + q : 4 * q + i)) * (4 * BITS));
+#pragma unroll
+                for (int k = 0; k < BITS; ++k) {
+                    __hip_atomic_fetch_and(ch + k, ~m[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_fetch_or(ch + k, b[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
             }
         }
     }
 }
 
 // The body of the compression kernels: workgroup wg of nwg takes 64-row groups wg, wg + nwg, ...
-template <int BITS, bool QJL, int MODE, int DT>
+// VALUES: a paged V tile in the values layout (no QJL); its own instance, so that the other layouts
+// carry none of its registers or LDS.
+template <int BITS, bool QJL, int MODE, int DT, bool VALUES>
 __device__ __forceinline__ void compress_rows(const CompressParams& p, int wg, int nwg) {
     constexpr int NC = 1 << BITS;
     constexpr int NB = NC - 1;
@@ -573,7 +591,65 @@ __device__ __forceinline__ void compress_rows(const CompressParams& p, int wg, i
     __shared__ uint2 s_cells[kCells];
     __shared__ int s_bad;
     // values layout: slices exchanged within each group of 4 rows (16 groups x 64 slices)
-    __shared__ __align__(16) uint32_t s_xchg[MODE == MODE_PAGED ? 1024 * (BITS == 3 ? 4 : BITS) : 1];
+    __shared__ __align__(16) uint32_t s_xchg[VALUES ? 1024 * (BITS == 3 ? 4 : BITS) : 1];
+    __shared__ uint2 s_slots[VALUES ? 256 : 1];  // the 64 slots around each wave's rows
+    // 1e-8 in the units of the unscaled rotation (paged mode)
+    const float den_eps = (MODE == MODE_PAGED && p.rotate) ? 1e-8f / p.wht_scale : 1e-8f;
+
+    // 16-bit paged rows run on the matrix cores (row l & 15 of the wave, lane group q = l >> 4);
+    // the others keep 4 consecutive lanes per row.  Either way the row's words leave lane q for
+    // dims 32q..32q+31.
+    constexpr bool GR = MODE == MODE_PAGED && DT != TQ_F32;
+    const int lane = threadIdx.x & 63;
+    const int q = GR ? (lane >> 4) : (threadIdx.x & 3);
+    const int row_in_wg = GR ? ((threadIdx.x >> 6) * 16 + (lane & 15)) : (threadIdx.x >> 2);  // 0..63
+
+    // Paged rows are head-major so that a workgroup's rows are consecutive tokens; each head's rows
+    // are padded to a multiple of 4.  row -> (token, head), false (and token 0, head 0) for padding
+    // and rows past the end.
+    auto locate = [&](int64_t row, int64_t& tok, int& head) -> bool {
+        bool ok = row >= 0 && row < p.n_rows;
+        if (p.idx32) {
+            const uint32_t r = ok ? (uint32_t)row : 0u, h = tq_udiv_apply(r, p.tok_div);
+            head = (int)h;
+            tok = r - h * (uint32_t)p.tok_rows;
+        } else {
+            const int64_t h = ok ? row / p.tok_rows : 0;
+            tok = ok ? row - h * p.tok_rows : 0;
+            head = (int)h;
+        }
+        ok = ok && tok < p.num_tokens;
+        tok = ok ? tok : 0;
+        head = ok ? head : 0;
+        return ok;
+    };
+    auto load_slot = [&](int64_t tok, uint32_t& lo, uint32_t& hi) {
+        const uint32_t* sp =
+            reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(p.slot_mapping) + tok * (p.slot_i64 ? 8 : 4));
+        lo = sp[0];
+        hi = sp[p.slot_i64 ? 1 : 0];
+    };
+    // Values layout: a chunk holds slots 4k..4k+3, and a token run seldom starts on a multiple of 4
+    // in a ragged batch.  So a wave's 16 rows move with the slots: a row that continues its
+    // predecessor's chunk (the next slot, not a multiple of 4) belongs to the wave of the chunk's
+    // first row.  The wave drops up to 3 such rows at its front and takes up to 3 past its end,
+    // which within one run leaves 16 rows in whole chunks; where runs meet, rows beyond 16 take a
+    // second pass.  link: bit l, row 16 w - 1 + l of the wave continues its predecessor, from one
+    // load of 64 slots a row group ahead.  16384 x 8, turbo4 K + V: one run off a multiple of 4
+    // 560 -> 21 us, 4 ragged sequences 137 -> 21 us (every row of such a run used to set its fields
+    // with atomics), an aligned run 21-22 us both ways.
+    const int64_t step = (int64_t)nwg * kRowsPerWG;
+    const int wave16 = __builtin_amdgcn_readfirstlane(16 * (int)(threadIdx.x >> 6));
+    // values: the next row group's slot window; else: the row's own slot (in flight either way while
+    // the row is quantised)
+    uint32_t slo = 0, shi = 0;
+    if (VALUES) {
+        int64_t tok;
+        int head;
+        locate((int64_t)wg * kRowsPerWG + wave16 + (lane - 1), tok, head);
+        load_slot(tok, slo, shi);
+    }
+
     if (threadIdx.x < NC) s_cent[threadIdx.x] = p.centroids[threadIdx.x];
     if (threadIdx.x == 0) s_bad = 0;
     // Boundaries are uniform: the loads below become scalar loads kept in SGPRs.
@@ -585,40 +661,46 @@ __device__ __forceinline__ void compress_rows(const CompressParams& p, int wg, i
     else build_cells<NB>(bd, p.boundaries, s_cells, &s_bad);
     __syncthreads();
     const bool cells = s_bad == 0;
-    // 1e-8 in the units of the unscaled rotation (paged mode)
-    const float den_eps = (MODE == MODE_PAGED && p.rotate) ? 1e-8f / p.wht_scale : 1e-8f;
-
-    // 16-bit paged rows run on the matrix cores (row l & 15 of the wave, lane group q = l >> 4);
-    // the others keep 4 consecutive lanes per row.  Either way the row's words leave lane q for
-    // dims 32q..32q+31.
-    constexpr bool GR = MODE == MODE_PAGED && DT != TQ_F32;
-    const int lane = threadIdx.x & 63;
-    const int q = GR ? (lane >> 4) : (threadIdx.x & 3);
-    const int row_in_wg = GR ? ((threadIdx.x >> 6) * 16 + (lane & 15)) : (threadIdx.x >> 2);  // 0..63
     HadamardFrags<DT> hf;
     if constexpr (GR) hf = hadamard_frags<DT>(lane);
 
-    for (int64_t row0 = (int64_t)wg * kRowsPerWG; row0 < p.n_rows; row0 += (int64_t)nwg * kRowsPerWG) {
-        const int64_t row = row0 + row_in_wg;
-        bool row_ok = row < p.n_rows;
-        // Paged rows are head-major so that a workgroup's rows are consecutive tokens; each
-        // head's rows are padded to a multiple of 4, so rows 4a..4a+3 (one 16-lane group of a
-        // wave) are tokens 4k..4k+3 of one head.
-        int64_t tok, head;
+    for (int64_t row0 = (int64_t)wg * kRowsPerWG; row0 < p.n_rows; row0 += step) {
+      uint64_t link = 0;
+      int first = 0, last = 16;  // the wave's rows, from its base
+      if (VALUES) {
+          int64_t wtok;
+          int whead;
+          const bool wok = locate(row0 + wave16 + (lane - 1), wtok, whead);
+          // (the lane before: wave_shr 1; lane 0's link is not used)
+          const uint32_t plo = __builtin_amdgcn_update_dpp(0, slo, 0x138, 0xf, 0xf, false);
+          bool next_slot = slo == plo + 1;
+          if (p.slot_i64) {
+              const uint32_t phi = __builtin_amdgcn_update_dpp(0, shi, 0x138, 0xf, 0xf, false);
+              next_slot = (((uint64_t)shi << 32) | slo) == (((uint64_t)phi << 32) | plo) + 1;
+          }
+          link = __builtin_amdgcn_ballot_w64(wok && wtok > 0 && next_slot && (slo & 3) != 0);
+          first = __builtin_ctzll(~(link >> 1));
+          last = 16 + __builtin_ctzll(~(link >> 17));
+          s_slots[threadIdx.x & (VALUES ? 255 : 0)] = make_uint2(slo, shi);
+          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+      }
+      for (int next; first < last; first = next) {
+        // a pass ends at a chunk: rows at its end that go on past 16 are left to the next one
+        next = first + 16;
+        if (VALUES && next < last) {
+            const int b = (int)(link >> (first + 15)) & 7;  // rows first + 14 .. first + 16 continue
+            next -= b == 7 ? 3 : (b >= 6 ? 2 : (b >= 4 ? 1 : 0));
+        }
+        const int end = next < last ? next : last;
+        const int64_t row = row0 + row_in_wg;  // MODE_UNPACKED
+        bool row_ok;
+        int64_t tok;
+        int head;
         if (MODE == MODE_PAGED) {
-            if (p.idx32) {
-                const uint32_t r = row_ok ? (uint32_t)row : 0u, nt = (uint32_t)p.tok_rows;
-                const uint32_t h = tq_udiv_apply(r, p.tok_div);
-                head = h;
-                tok = r - h * nt;
-            } else {
-                head = row_ok ? row / p.tok_rows : 0;
-                tok = row_ok ? row - head * p.tok_rows : 0;
-            }
-            row_ok = row_ok && tok < p.num_tokens;
-            tok = row_ok ? tok : 0;
-            head = row_ok ? head : 0;
+            row_ok = locate(row0 + wave16 + (first + (row_in_wg & 15)), tok, head) && (!VALUES || first + (row_in_wg & 15) < end);
         } else {
+            row_ok = row < p.n_rows;
             head = 0;
             tok = row_ok ? row : 0;
         }
@@ -628,18 +710,16 @@ __device__ __forceinline__ void compress_rows(const CompressParams& p, int wg, i
         int64_t off;
         const uint32_t lane_off = GR ? 8u * q : 32u * q;
         if (p.idx32) off = (uint32_t)tok * (uint32_t)p.x_stride_token + (uint32_t)head * (uint32_t)p.x_stride_head + lane_off;
-        else off = tok * p.x_stride_token + head * p.x_stride_head + lane_off;
+        else off = tok * p.x_stride_token + (int64_t)head * p.x_stride_head + lane_off;
         RawRow<DT> raw;
         if constexpr (GR) load_raw_groups<DT>(p.x, off, raw);
         else load_raw<DT>(p.x, off, raw);
         // the slot goes out with the row (token 0's for rows that are not written, whose result
         // is dropped): its round trip overlaps the row's instead of following the quantisation
-        uint32_t slo = 0, shi = 0;
         if (MODE == MODE_PAGED) {
-            const uint32_t* sp = reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(p.slot_mapping) +
-                                                                   tok * (p.slot_i64 ? 8 : 4));
-            slo = sp[0];
-            shi = sp[p.slot_i64 ? 1 : 0];
+            int wh;
+            if (VALUES) locate(row0 + step + wave16 + (lane - 1), tok, wh);
+            load_slot(tok, slo, shi);
         }
         float v[32];
         float norm, den, rcp;
@@ -705,8 +785,11 @@ __device__ __forceinline__ void compress_rows(const CompressParams& p, int wg, i
 #pragma unroll
                 for (int k = 0; k < 32; ++k) idx[k] = quant_cell(v[k], s_cells);
             } else {
+                float bl[NB];  // read again: this path is rare, and bd would hold its registers through the loop
 #pragma unroll
-                for (int k = 0; k < 32; ++k) idx[k] = quant_linear<NB>(v[k], bd);
+                for (int i = 0; i < NB; ++i) bl[i] = p.boundaries[i];
+#pragma unroll
+                for (int k = 0; k < 32; ++k) idx[k] = quant_linear<NB>(v[k], bl);
             }
             if (QJL) {
                 float r[32];
@@ -739,8 +822,10 @@ __device__ __forceinline__ void compress_rows(const CompressParams& p, int wg, i
                 }
             }
         } else {
+            uint2 sw = make_uint2(slo, shi);
+            if (VALUES) sw = s_slots[((threadIdx.x & ~63) + first + (row_in_wg & 15) + 1) & (VALUES ? 255 : 0)];
             const int64_t slot =
-                !row_ok ? -1 : (p.slot_i64 ? (int64_t)(((uint64_t)shi << 32) | slo) : (int64_t)(int32_t)slo);
+                !row_ok ? -1 : (p.slot_i64 ? (int64_t)(((uint64_t)sw.y << 32) | sw.x) : (int64_t)(int32_t)sw.x);
             const bool write = row_ok && slot >= 0 && slot < p.num_blocks * p.block_size;
             int64_t blk, r_in_blk;
             if (p.idx32) {
@@ -752,11 +837,18 @@ __device__ __forceinline__ void compress_rows(const CompressParams& p, int wg, i
                 blk = write ? slot / p.block_size : 0;
                 r_in_blk = write ? slot - blk * p.block_size : 0;
             }
-            uint8_t* tile = p.cache + blk * p.stride_block + head * p.stride_head;
-            if (p.tile_layout == TQ_TILE_VALUES) {
+            uint8_t* tile = p.cache + blk * p.stride_block + (int64_t)head * p.stride_head;
+            if (VALUES) {
+                // rows lead_row .. lead_row + 3 of the pass are slots 4k..4k+3
+                const int r16 = row_in_wg & 15, pos = (int)(sw.x & 3), lead_row = r16 - pos;
+                const uint32_t plink = (uint32_t)(link >> (first + 1)) & 0x7ffffu;  // bit r: row r continues row r - 1
+                const bool full = write && lead_row >= 0 && lead_row <= 12 && first + lead_row + 3 < end &&
+                                  ((plink >> ((lead_row + 1) & 31)) & 7) == 7;
+                const uint64_t leaders = __builtin_amdgcn_ballot_w64(full && pos == 0 && q == 0);
+                const int gi = __builtin_popcountll(leaders & ((1ull << ((GR ? lead_row : 4 * lead_row) & 63)) - 1));
                 if (BITS >= 2)
-                    store_values<BITS < 2 ? 2 : BITS, GR>(value_slices<BITS < 2 ? 2 : BITS>(idx), write, slot, tile,
-                                                          r_in_blk, q, s_xchg);
+                    store_values<BITS < 2 ? 2 : BITS, GR>(value_slices<BITS < 2 ? 2 : BITS>(idx), write, full, gi, r16, end - first,
+                                                          plink, tile, r_in_blk, q, s_xchg);
                 if (write && q == 0)
                     *reinterpret_cast<uint16_t*>(tile + p.off_norm + r_in_blk * p.rs_norm) = (uint16_t)tq_f32_to_f16_bits(norm);
                 continue;
@@ -808,30 +900,43 @@ __device__ __forceinline__ void compress_rows(const CompressParams& p, int wg, i
                 }
             }
         }
+      }
     }
 }
 
-// Resident waves per SIMD the kernel is compiled for: the matrix-core rows (16-bit paged input)
-// without QJL fit 4 (128 registers: the Hadamard fragments, the accumulators and the row), the
-// others keep the compiler's own choice.
-template <int MODE, int DT, bool QJL>
+template <int BITS, bool QJL, int MODE, int DT>
+__device__ __forceinline__ void compress_any(const CompressParams& p, int wg, int nwg) {
+    if constexpr (MODE == MODE_PAGED && !QJL && BITS >= 2) {
+        if (p.tile_layout == TQ_TILE_VALUES) {
+            compress_rows<BITS, QJL, MODE, DT, true>(p, wg, nwg);
+            return;
+        }
+    }
+    compress_rows<BITS, QJL, MODE, DT, false>(p, wg, nwg);
+}
+
+// Resident waves per SIMD the paged kernels are compiled for: 4 (128 registers); 3 with QJL keys of 2
+// and 3 bits (the residual row; left to itself the compiler parked 32 registers in AGPRs and ran 2
+// waves: 16384 x 8 turbo3 + QJL / turbo3 25.8 -> 23.1 us, turbo2 + QJL / turbo2 25.2 -> 21.4 us);
+// turbo4 + QJL keeps 2 (3 would spill 12 registers: 25.8 against 26.8 us).
+template <int BITS, int MODE, bool QJL>
 constexpr int compress_min_waves() {
-    return (MODE == MODE_PAGED && DT != TQ_F32 && !QJL) ? 4 : 1;
+    return MODE != MODE_PAGED ? 1 : (!QJL ? 4 : (BITS < 4 ? 3 : 1));
 }
 
 template <int BITS, bool QJL, int MODE, int DT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(compress_min_waves<MODE, DT, QJL>(), 8)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(compress_min_waves<BITS, MODE, QJL>(), 8)))
 void compress_kernel(CompressParams p) {
-    compress_rows<BITS, QJL, MODE, DT>(p, blockIdx.x, gridDim.x);
+    compress_any<BITS, QJL, MODE, DT>(p, blockIdx.x, gridDim.x);
 }
 
 // K and V of one layer in one launch (same bits; V without QJL): workgroups [0, gk) take K, the
 // rest V.  One launch instead of two halves the fixed cost of a K + V cache update.
 template <int BITS, bool QJL_K, int DT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(compress_min_waves<MODE_PAGED, DT, QJL_K>(), 8)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(compress_min_waves<BITS, MODE_PAGED, QJL_K>(), 8)))
 void compress_kv_kernel(CompressParams pk, CompressParams pv, int gk) {
-    if ((int)blockIdx.x < gk) compress_rows<BITS, QJL_K, MODE_PAGED, DT>(pk, blockIdx.x, gk);
-    else compress_rows<BITS, false, MODE_PAGED, DT>(pv, blockIdx.x - gk, gridDim.x - gk);
+    if ((int)blockIdx.x < gk) compress_any<BITS, QJL_K, MODE_PAGED, DT>(pk, blockIdx.x, gk);
+    else compress_any<BITS, false, MODE_PAGED, DT>(pv, blockIdx.x - gk, gridDim.x - gk);
 }
 
 template <int MODE>
@@ -1101,13 +1206,17 @@ extern "C" int tq_compress_paged_kv(const tq_paged_target* k, const tq_paged_tar
         rc = launch_compress<MODE_PAGED>(pk, k->bits, k->use_qjl, st);
         return rc ? rc : launch_compress<MODE_PAGED>(pv, v->bits, v->use_qjl, st);
     }
-    // K workgroups first, then as many V workgroups: half the resident workgroups each
+    // K workgroups first, then the V workgroups: of the resident workgroups 29 / 64 take K and the
+    // rest V.  A V wave has the extra pass where runs meet; with halves it was the last to end
+    // (16384 x 8, one run off a multiple of 4: turbo4 28.8 against 20.9 us, turbo3 + QJL 45.0 against
+    // 26.0 us; an aligned run 21.2 against 21.7 us).
     const int64_t groups = (pk.n_rows + kRowsPerWG - 1) / kRowsPerWG;
 #define TQ_KV_DT(B, Q, DT)                                                                          \
     do {                                                                                            \
         static const int res = resident_grid(compress_kv_kernel<B, Q, DT>) / 2;                     \
         const int gk = (int)(groups < res ? groups : (res > 0 ? res : 1));                          \
-        hipLaunchKernelGGL((compress_kv_kernel<B, Q, DT>), dim3(2 * gk), dim3(256), 0, st, pk, pv, gk); \
+        hipLaunchKernelGGL((compress_kv_kernel<B, Q, DT>), dim3(2 * gk), dim3(256), 0, st, pk, pv,     \
+                           groups > gk ? gk * 29 / 32 : gk);                                        \
     } while (0)
 #define TQ_KV(B, Q)                                             \
     do {                                                        \
