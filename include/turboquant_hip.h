@@ -383,6 +383,15 @@ int tq_prefill(const void* q, int q_dtype, int64_t q_stride_token, int64_t q_str
 
 size_t tq_decode_workspace_bytes(int num_seqs, int num_q_heads, int max_seq_len, int tokens_per_chunk);
 
+/* Workspace with which tq_decode runs a Sparse-V call of one chunk per sequence (tokens_per_chunk >=
+ * max_seq_len, the reference's single pass, kernels/sparse_v.py:316,341) on the general layouts over
+ * several units per (sequence, KV head), with the single pass's running max and skipped tokens: a first
+ * pass leaves every unit's score maxima there.  With less than this (and at least
+ * tq_decode_workspace_bytes) the call is one unit per (sequence, KV head).  Equal to
+ * tq_decode_workspace_bytes for calls that are never split. */
+size_t tq_decode_sparse_workspace_bytes(int num_seqs, int num_q_heads, int num_kv_heads, int max_seq_len,
+                                        int tokens_per_chunk);
+
 /*
  * tq_decode without a caller workspace and without any device allocation: the split-K partial
  * results go to a fixed array of TQ_NOALLOC_SCRATCH_BYTES inside this library (one copy per

@@ -77,6 +77,8 @@ struct DecodeParams {
     float* ws_acc;     // [num_seqs][hq][n_chunks][128]
     float* ws_m;       // [num_seqs][hq][n_chunks]  (log2 domain)
     float* ws_l;
+    float* ws_pm;      // split single pass: [num_seqs][hq][n_chunks] score maxima (log2 domain), or null
+    int len_limit;     // tokens of a sequence that are processed
     unsigned long long* skip_stats;
     void* out;
     int out_dtype;
@@ -442,7 +444,9 @@ constexpr int decode_waves() {
     return (!QCOLS && KQJL && VB == 3 && KB >= 3) ? 2 : 3;
 }
 
-template <int KB, bool KQJL, int VB, bool QCOLS, bool NV>
+// MAXP: the first of the two passes of a split Sparse-V single pass (launched with VB = KB): only the
+// scores' maxima of each unit, per query head, go to ws_pm (the values are not read).
+template <int KB, bool KQJL, int VB, bool QCOLS, bool NV, bool MAXP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(decode_waves<KB, KQJL, VB, QCOLS>(),
                                                                      decode_waves<KB, KQJL, VB, QCOLS>())))
 void decode_kernel(DecodeParams p) {
@@ -452,7 +456,7 @@ void decode_kernel(DecodeParams p) {
     // table goes first, so each table's address is a multiple of its size (see pair_addr).
     // K and V share one table when they use the same codebook (p.share_tab).
     extern __shared__ uint32_t s_lds[];
-    uint32_t* s_ktab = (KENT >= VENT || p.share_tab) ? s_lds : s_lds + VENT * 32;
+    uint32_t* s_ktab = (KENT >= VENT || p.share_tab || MAXP) ? s_lds : s_lds + VENT * 32;
     uint32_t* s_vtab = p.share_tab ? s_lds : (KENT >= VENT ? s_lds + KENT * 32 : s_lds);
 
     // Pair tables: entry e -> half2(c[e & (2^b - 1)], c[e >> b]) * cscale, 32 bank replicas.
@@ -460,7 +464,7 @@ void decode_kernel(DecodeParams p) {
         int e = i >> 5;
         s_ktab[i] = tq_pack_half2(p.k_cent[e & ((1 << KB) - 1)] * p.k_cscale, p.k_cent[e >> KB] * p.k_cscale);
     }
-    if (!p.share_tab) {
+    if (!p.share_tab && !MAXP) {
         for (int i = threadIdx.x; i < VENT * 32; i += 256) {
             int e = i >> 5;
             s_vtab[i] = tq_pack_half2(p.v_cent[e & ((1 << VB) - 1)] * p.v_cscale, p.v_cent[e >> VB] * p.v_cscale);
@@ -492,6 +496,7 @@ void decode_kernel(DecodeParams p) {
     int L = tq_seq_len(p.seq_lens, s, p.uniform_len);
     const int cap = p.max_blocks * p.block_size;
     L = L < cap ? L : cap;
+    L = L < p.len_limit ? L : p.len_limit;
     const int t_begin = c * p.chunk;
     if (t_begin >= L) return;
     const int t_end = (t_begin + p.chunk < L) ? t_begin + p.chunk : L;
@@ -633,8 +638,50 @@ void decode_kernel(DecodeParams p) {
             tl.base[r] = ub[r] + (r >= R_VIDX ? offv : offk) + (int64_t)rowbase * p.rrow[r];
     };
 
+    const int ntiles = (t_end - t_begin + 15) >> 4;
+    const int nfull = (t_end - t_begin) >> 4;
+    const int nload = paged ? ntiles : nfull;
+    if constexpr (MAXP) {
+        // keys only, so four tiles fit in flight
+        constexpr int DM = 4;
+        TileRaw<KB, KQJL, VB, NV> ring[DM];
+        int nv[DM];
+        auto fetch = [&](int k, TileRaw<KB, KQJL, VB, NV>& raw, int& nvalid) {
+            Tile tl;
+            locate(t_begin + 16 * k, k < nload, tl);
+            nvalid = tl.nvalid;
+            load_tile<KB, KQJL, VB, NV, false>(raw, tl, o, p.rrow, p.vstep, NV && p.v_lg);
+        };
+        float m = kNegInf, sc[4];
+#pragma unroll
+        for (int k = 0; k < DM - 1; ++k) fetch(k, ring[k], nv[k]);
+        for (int i = 0; i < nload; i += DM) {
+#pragma unroll
+            for (int k = 0; k < DM; ++k) {
+                fetch(i + k + DM - 1, ring[(k + DM - 1) % DM], nv[(k + DM - 1) % DM]);
+                // (a tile past the end has no valid row: -inf)
+                m = fmaxf(m, tile_scores<KB, KQJL, VB, NV, QCOLS, false>(ring[k], nv[k], qop, qlo, qpop, qpm, kbank, one, g,
+                                                                         sc));
+            }
+        }
+        if (nload < ntiles) {
+            Tile tl;
+            locate(t_begin + 16 * nfull, true, tl);
+            TileRaw<KB, KQJL, VB, NV> tr;
+            load_tile<KB, KQJL, VB, NV, true>(tr, tl, o, p.rrow, p.vstep, NV && p.v_lg);
+            m = fmaxf(m, tile_scores<KB, KQJL, VB, NV, QCOLS, false>(tr, tl.nvalid, qop, qlo, qpop, qpm, kbank, one, g, sc));
+        }
+        if (hvalid && g == 0) p.ws_pm[(s * p.hq + head) * (int64_t)p.n_chunks + c] = m;
+        return;
+    }
     SoftmaxState sm;
     sm.m = kNegInf;
+    if (p.ws_pm && c > 0) {
+        // the running max as the single pass has it here: the maxima of the units before
+        const float* pm = p.ws_pm + (s * p.hq + (hvalid ? head : kh * p.group)) * (int64_t)p.n_chunks;
+        for (int cb = g; cb < c; cb += 4) sm.m = fmaxf(sm.m, pm[cb]);
+        sm.m = hvalid ? max_over_groups(sm.m) : kNegInf;
+    }
     sm.lsum = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) sm.acc[i] = tq_floatx4{0.f, 0.f, 0.f, 0.f};
@@ -661,9 +708,6 @@ void decode_kernel(DecodeParams p) {
     static_assert(D == 2, "the KV-block max look-ahead reads the next tile from the other ring slot");
     const bool blk2 = sparse && p.sparse_pair;  // (paged: the partial last tile is in the ring)
     float m_blk = kNegInf;
-    const int ntiles = (t_end - t_begin + 15) >> 4;
-    const int nfull = (t_end - t_begin) >> 4;
-    const int nload = paged ? ntiles : nfull;
     TileRaw<KB, KQJL, VB, NV> ring[D];
     int nv[D];
 #pragma unroll
@@ -934,15 +978,54 @@ size_t lds_bytes(int kb, int vb, int share) {
 const void* decode_kernel_ptr(int kb, bool kq, int vb, bool qcols, bool nv) {
 #define TQ_KP(KB, KQ, VB)                                                                          \
     if (kb == KB && kq == KQ && vb == VB)                                                          \
-        return qcols ? (nv ? (const void*)decode_kernel<KB, KQ, VB, true, true>                    \
-                           : (const void*)decode_kernel<KB, KQ, VB, true, false>)                  \
-                     : (nv ? (const void*)decode_kernel<KB, KQ, VB, false, true>                   \
-                           : (const void*)decode_kernel<KB, KQ, VB, false, false>);
+        return qcols ? (nv ? (const void*)decode_kernel<KB, KQ, VB, true, true, false>             \
+                           : (const void*)decode_kernel<KB, KQ, VB, true, false, false>)           \
+                     : (nv ? (const void*)decode_kernel<KB, KQ, VB, false, true, false>            \
+                           : (const void*)decode_kernel<KB, KQ, VB, false, false, false>);
 #define TQ_KP_V(KB, KQ) TQ_KP(KB, KQ, 2) TQ_KP(KB, KQ, 3) TQ_KP(KB, KQ, 4)
     TQ_KP_V(2, false) TQ_KP_V(2, true) TQ_KP_V(3, false) TQ_KP_V(3, true) TQ_KP_V(4, false) TQ_KP_V(4, true)
 #undef TQ_KP_V
 #undef TQ_KP
     return nullptr;
+}
+
+// The instance that writes the units' score maxima (first pass of a split single pass).
+const void* decode_max_kernel_ptr(int kb, bool kq, bool qcols, bool nv) {
+#define TQ_KM(KB, KQ)                                                                              \
+    if (kb == KB && kq == KQ)                                                                      \
+        return qcols ? (nv ? (const void*)decode_kernel<KB, KQ, KB, true, true, true>              \
+                           : (const void*)decode_kernel<KB, KQ, KB, true, false, true>)            \
+                     : (nv ? (const void*)decode_kernel<KB, KQ, KB, false, true, true>             \
+                           : (const void*)decode_kernel<KB, KQ, KB, false, false, true>);
+    TQ_KM(2, false) TQ_KM(2, true) TQ_KM(3, false) TQ_KM(3, true) TQ_KM(4, false) TQ_KM(4, true)
+#undef TQ_KM
+    return nullptr;
+}
+
+// Split of a Sparse-V single pass (one unit per (sequence, KV head)) over n units per (sequence,
+// KV head) of *chunk tokens each (a multiple of 32, the longest KV block the running max follows).
+// The skip test of a unit needs only the running max at its start, so a first pass over the keys
+// leaves every unit's maxima and the second pass starts from the maxima before it: the same
+// skipped tokens as one pass.  Worth the second reading of the keys while the units of one pass
+// are fewer than a third of the waves that fit the device; a unit has at least kSplitTiles tiles,
+// about its start-up.  Returns 1 where it stays one pass.  A single pass is a serial chain of ~1.3 us
+// per tile; 24 / 4 heads, turbo3, block 32, one pass against split: 8 x 4096 tokens 341 / 32.6 us,
+// 1 x 16384 1345 / 33.5 us, 1 x 1024 92 / 25 us, 64 x 2048 (8 units each) 181 / 59 us.
+constexpr int kSplitWaves = 256 * 4 * 2;  // CUs x SIMDs x 2
+constexpr int kSplitTiles = 4;
+int single_pass_split(int num_seqs, int num_kv_heads, int limit, int* chunk) {
+    const int64_t units = (int64_t)num_seqs * num_kv_heads;
+    const int64_t pairs = ((int64_t)limit + 31) / 32;
+    int64_t n = kSplitWaves / (units > 0 ? units : 1);
+    n = n < pairs * 2 / kSplitTiles ? n : pairs * 2 / kSplitTiles;
+    if (n < 3) return 1;
+    const int64_t per = (pairs + n - 1) / n;
+    *chunk = (int)(32 * per);
+    return (int)((pairs + per - 1) / per);
+}
+size_t split_bytes(int num_seqs, int num_q_heads, int n) {
+    const size_t slots = (size_t)num_seqs * num_q_heads * n;
+    return align_up(slots * TQ_HEAD_DIM * sizeof(float), 256) + 3 * align_up(slots * sizeof(float), 256);
 }
 
 bool q_vector_ok(const void* q, int dtype, int64_t ss, int64_t sh) {
@@ -1116,6 +1199,16 @@ extern "C" size_t tq_decode_workspace_bytes(int num_seqs, int num_q_heads, int m
     return align_up(slots * TQ_HEAD_DIM * sizeof(float), 256) + 2 * align_up(slots * sizeof(float), 256);
 }
 
+extern "C" size_t tq_decode_sparse_workspace_bytes(int num_seqs, int num_q_heads, int num_kv_heads, int max_seq_len,
+                                                   int tokens_per_chunk) {
+    const size_t need = tq_decode_workspace_bytes(num_seqs, num_q_heads, max_seq_len, tokens_per_chunk);
+    if (need == 0 || num_kv_heads <= 0 || tokens_per_chunk < max_seq_len || max_seq_len <= 0) return need;
+    int chunk = 0;
+    const int n = single_pass_split(num_seqs, num_kv_heads, max_seq_len, &chunk);
+    const size_t split = n > 1 ? split_bytes(num_seqs, num_q_heads, n) : 0;
+    return split > need ? split : need;
+}
+
 extern "C" int tq_decode_concurrent_units(int k_bits, int k_qjl, int v_bits, int num_q_heads, int num_kv_heads,
                                           int norm_row_bytes, int share_codebook, int* units) {
     if (!units) return TQ_ERR_INVALID_ARGUMENT;
@@ -1269,7 +1362,25 @@ int tq_decode_impl(int rotate, const void* q, int q_dtype, int64_t q_stride_seq,
     if (tokens_per_chunk == 0 && !fast)
         tokens_per_chunk = general_chunk(num_seqs, num_q_heads, max_seq_len, sparse_pair);
     if (!balanced && sparse_pair && tokens_per_chunk % 32) tokens_per_chunk += 16;
-    const int n_chunks = balanced ? 1 : n_chunks_for(max_seq_len, tokens_per_chunk);
+    int n_chunks = balanced ? 1 : n_chunks_for(max_seq_len, tokens_per_chunk);
+    // tokens of a sequence that the call processes
+    const int64_t span = balanced ? bal_cap : (int64_t)n_chunks * tokens_per_chunk;
+    const int len_limit = (int)(span < bal_cap ? span : bal_cap);
+    bool split = false;
+    if (!fast && !contig && n_chunks == 1 && sparse_threshold > 0.f && max_seq_len > 0 &&
+        workspace_bytes >= tq_decode_sparse_workspace_bytes(num_seqs, num_q_heads, num_kv_heads, max_seq_len,
+                                                            tokens_per_chunk)) {
+        // (units past max_seq_len, for sequences longer than it that the single pass would still
+        // take up to len_limit, must fit too; otherwise it stays one pass)
+        int chunk = 0;
+        const int n = single_pass_split(num_seqs, num_kv_heads, max_seq_len, &chunk);
+        const int n_all = n > 1 ? (len_limit + chunk - 1) / chunk : 1;
+        if (n > 1 && split_bytes(num_seqs, num_q_heads, n_all) <= workspace_bytes) {
+            split = true;
+            tokens_per_chunk = chunk;
+            n_chunks = n_all;
+        }
+    }
 
     const size_t slots = (size_t)num_seqs * num_q_heads * n_chunks;
     uint8_t* ws = static_cast<uint8_t*>(workspace);
@@ -1429,9 +1540,12 @@ int tq_decode_impl(int rotate, const void* q, int q_dtype, int64_t q_stride_seq,
     p.sparse_pair = sparse_pair ? 1 : 0;
     p.chunk = tokens_per_chunk;
     p.n_chunks = n_chunks;
+    p.len_limit = len_limit;
     p.ws_acc = ws_acc;
     p.ws_m = ws_m;
     p.ws_l = ws_l;
+    p.ws_pm = split ? reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(ws_l) + align_up(slots * sizeof(float), 256))
+                    : nullptr;
     p.skip_stats = skip_stats;
     p.out = out;
     p.out_dtype = out_dtype;
@@ -1454,14 +1568,19 @@ int tq_decode_impl(int rotate, const void* q, int q_dtype, int64_t q_stride_seq,
     const void* kern = decode_kernel_ptr(k->bits, k->qjl != 0, v->bits, group <= 8, nv);
     if (!kern) return TQ_ERR_BITS;
     void* args[] = {&p};
+    if (split) {
+        const void* kmax = decode_max_kernel_ptr(k->bits, k->qjl != 0, group <= 8, nv);
+        if (!kmax) return TQ_ERR_BITS;
+        const hipError_t me = hipLaunchKernel(kmax, dim3((unsigned)grid), dim3(256), args, lds_bytes(k->bits, k->bits, 1), st);
+        if (me != hipSuccess) return (int)me;
+    }
     hipError_t le = hipLaunchKernel(kern, dim3((unsigned)grid), dim3(256), args,
                                     lds_bytes(k->bits, v->bits, p.share_tab), st);
     if (le != hipSuccess) return (int)le;
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
 
-    return launch_reduce(ws_acc, ws_m, ws_l, num_seqs, num_q_heads, n_chunks, tokens_per_chunk,
-                         max_blocks_per_seq * block_size, seq_lens, max_seq_len, out, out_dtype, out_stride_seq, out_stride_head,
+    return launch_reduce(ws_acc, ws_m, ws_l, num_seqs, num_q_heads, n_chunks, tokens_per_chunk, len_limit, seq_lens, max_seq_len, out, out_dtype, out_stride_seq, out_stride_head,
                          rotate, st);
 }
 

@@ -135,6 +135,7 @@ SIGNATURES = {
          _f32, _f32, _i32, _vp, _i32, _i64, _i64, _vp],
     ),
     "tq_decode_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32]),
+    "tq_decode_sparse_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32, _i32]),
     "tq_decode_noalloc": (
         _i32,
         [_vp, _i32, _i64, _i64, _vp, _i64, _i64, _i32, _i32, _i32, _i32,

@@ -525,6 +525,9 @@ def run_decode(
     L = _lib.lib()
     need = L.tq_decode_workspace_bytes(S, Hq, max_seq_len, tokens_per_chunk)
     if workspace is None or workspace.numel() < need or workspace.data_ptr() % 256:
+        if sparse_threshold > 0:
+            # room for a split single pass (a caller's own workspace decides that by its size)
+            need = L.tq_decode_sparse_workspace_bytes(S, Hq, num_kv_heads, max_seq_len, tokens_per_chunk)
         workspace = decode_workspace(dev, need)
     if skip_stats is not None and (skip_stats.dtype != torch.int64 or skip_stats.numel() < 2 or not skip_stats.is_cuda):
         raise ValueError("skip_stats must be a device int64 tensor with 2 elements")
