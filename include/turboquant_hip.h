@@ -381,6 +381,27 @@ int tq_prefill(const void* q, int q_dtype, int64_t q_stride_token, int64_t q_str
                void* out, int out_dtype, int64_t out_stride_token, int64_t out_stride_head,
                tq_stream_t stream);
 
+/*
+ * tq_prefill with a workspace of tq_prefill_workspace_bytes(...), 256-byte aligned (no initial contents
+ * needed; calls that overlap in time must not share one): the key tokens of all row blocks are then
+ * shared equally by the device's waves, a row block's keys over several waves where needed, and the
+ * pieces merged.  A null or smaller workspace gives tq_prefill.  Same arguments, checks and results
+ * otherwise.
+ */
+int tq_prefill_split(const void* q, int q_dtype, int64_t q_stride_token, int64_t q_stride_head,
+                     const void* q_proj, int64_t qp_stride_token, int64_t qp_stride_head,
+                     const int32_t* cu_seqlens_q, int num_seqs, int max_q_len,
+                     int num_q_heads, int num_kv_heads, int head_dim,
+                     const tq_kv_view* k, const tq_kv_view* v,
+                     int block_size, int64_t num_blocks,
+                     const int32_t* block_tables, int64_t block_table_stride, int max_blocks_per_seq,
+                     const int32_t* seq_lens, float sm_scale, float corr_scale, int flags,
+                     void* workspace, size_t workspace_bytes,
+                     void* out, int out_dtype, int64_t out_stride_token, int64_t out_stride_head,
+                     tq_stream_t stream);
+size_t tq_prefill_workspace_bytes(int num_seqs, int max_q_len, int num_q_heads, int num_kv_heads,
+                                  int max_blocks_per_seq, int block_size);
+
 size_t tq_decode_workspace_bytes(int num_seqs, int num_q_heads, int max_seq_len, int tokens_per_chunk);
 
 /* Workspace with which tq_decode runs a Sparse-V call of one chunk per sequence (tokens_per_chunk >=

@@ -183,3 +183,45 @@ def test_prefill_last_row_is_a_decode_step(dev):
             hs = slice(kh * G, (kh + 1) * G)
             want = odec.decode_dense(qr[i, hs], qr[i, hs], k[:i + 1], sg[:i + 1], rn[:i + 1], v[:i + 1], SM, CS)
             np.testing.assert_allclose(got[i, hs], want, rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("kb", [2, 3, 4])
+@pytest.mark.parametrize("kq", [False, True])
+@pytest.mark.parametrize("vb,G", [(2, 16), (3, 1), (4, 5)])
+def test_prefill_stream_formats(dev, kb, kq, vb, G):
+    """Every pair of formats of the streaming kernel, on segments that are cut over several waves and
+    merged (1000 and 340 tokens, few rows) next to short and empty ones."""
+    Hkv, bs = 2, 48
+    lens, n_new = [1000, 0, 340, 1, 31], [3, 2, 40, 1, 0]
+    case = build_case(40 + 9 * kb + vb + G, len(lens), G * Hkv, Hkv, lens, kb, kq, vb, bs)
+    q, cu = make_queries(np.random.default_rng(G), n_new, G * Hkv)
+    got, qr, _ = run_prefill(dev, case, q, cu, kb, kq, vb, bs, SM, CS, max_q_len=40)
+    want = oracle_prefill(case, qr, cu, G * Hkv, Hkv, kb, kq, vb, SM, CS)
+    np.testing.assert_allclose(got, want, rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("workspace", [True, False])
+@pytest.mark.parametrize("name", ["many", "long", "full"])
+def test_prefill_stream_shares(dev, monkeypatch, name, workspace, causal):
+    """The streaming kernel's ways to share out segments against prefill_kernel (which a separate q_proj
+    selects): more sequences than a wave's lanes, each segment whole; one long sequence over all
+    waves; more segments than waves; each also without a workspace.  Both are within RTOL / ATOL of the
+    oracle, so within twice that of each other."""
+    from turboquant import _lib
+    kb, kq, vb, Hkv, bs = 3, True, 3, 8, 16
+    rng = np.random.default_rng(2)
+    if name == "many":
+        G, lens = 3, [int(x) for x in rng.integers(0, 200, 70)] + [200]
+        n_new = [int(x) for x in rng.integers(0, 40, 71)]
+    elif name == "long":
+        G, lens, n_new = 4, [6000], [50]
+    else:
+        G, lens, n_new = 16, [30, 850], [9, 800]
+    case = build_case(7, len(lens), G * Hkv, Hkv, lens, kb, kq, vb, bs)
+    q, cu = make_queries(rng, n_new, G * Hkv)
+    want, _, _ = run_prefill(dev, case, q, cu, kb, kq, vb, bs, SM, CS, qp=q, causal=causal, out_dtype=torch.float32)
+    if not workspace:
+        monkeypatch.setattr(_lib.lib(), "tq_prefill_workspace_bytes", lambda *a: 0)
+    got, _, _ = run_prefill(dev, case, q, cu, kb, kq, vb, bs, SM, CS, causal=causal, out_dtype=torch.float32)
+    np.testing.assert_allclose(got, want, rtol=2 * RTOL, atol=2 * ATOL)

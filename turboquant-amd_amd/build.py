@@ -50,6 +50,7 @@ COMMON_FLAGS = [
 # -inf, never NaN), so fmax needs no quieting of its operands.
 FILE_FLAGS = {
     "tq_decode_fast.hip": ["-fno-honor-nans"],
+    "tq_prefill_stream.hip": ["-fno-honor-nans"],
 }
 
 

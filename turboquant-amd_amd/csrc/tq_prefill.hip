@@ -3,7 +3,8 @@
 // one online softmax per query row over 16x128 key tiles, fp16 MFMA products with fp32
 // accumulation), reading the packed paged cache directly instead of dequantised arrays, with
 // the causal limit of a serving extend step (query i of a sequence of length L with n new
-// tokens sits at position L - n + i and sees keys 0 .. L - n + i).
+// tokens sits at position L - n + i and sees keys 0 .. L - n + i).  prefill_kernel serves what
+// prefill_stream_kernel does not take (stream_ok and the conditions at its launch).
 //
 // Workgroup (256 threads, 4 waves) = (sequence s, KV head kh, block of 128 rows); a row is one
 // (new token i, query head of the GQA group) pair, rows ordered token-major, so a workgroup
@@ -29,8 +30,10 @@
 //   O^T [128 x 16 rows] += VhatT . P^T        8 x mfma_f32_16x16x32_f16 per step
 // Output: lane (n, g) holds dims 16j + 4g + r of row n, divided by the row's denominator.
 #include "tq_common.h"
+#include "tq_prefill_internal.h"
 
 #include <cmath>
+#include <mutex>
 
 namespace {
 
@@ -543,9 +546,59 @@ bool q_vector_ok(const void* q, int dtype, int64_t st, int64_t sh) {
     return aligned(q, a) && st % 8 == 0 && sh % 8 == 0;
 }
 
-}  // namespace
+// Compute units of the current device (cached per device).
+int device_cus(int* cus) {
+    static int cache[64];
+    static std::mutex mu;
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return (int)e;
+    std::lock_guard<std::mutex> lock(mu);
+    if (dev < 64 && cache[dev] > 0) {
+        *cus = cache[dev];
+        return TQ_OK;
+    }
+    e = hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e != hipSuccess) return (int)e;
+    if (dev < 64) cache[dev] = *cus;
+    return TQ_OK;
+}
 
-extern "C" int tq_prefill(const void* q, int q_dtype, int64_t q_stride_token, int64_t q_stride_head,
+// Workers of prefill_stream_kernel that a call can use at most (256 CUs x 8 waves, each at least 128
+// tokens of the stream), and the workspace for their pieces (two per
+// worker) and the cuts' plan.
+constexpr int64_t kStreamWorkers = 256 * kTqPrefillStreamWaves;
+// Block tables of at most this many tokens stay with prefill_kernel: its start is shorter, a workgroup's
+// walk longer (32 query heads on 8 KV heads, 3-bit keys with QJL, no earlier tokens, one / 16 sequences:
+// 32 tokens 18 / 18 us here, 20 / 23 there; 128 tokens 25 / 37 and 27 / 39; 512 tokens after 512 earlier
+// ones 90 / - and 58 / -; one of 640 tokens 62 and 33).
+constexpr int64_t kStreamMinTokens = 192;
+int64_t stream_workers(int num_seqs, int max_q_len, int num_q_heads, int num_kv_heads, int64_t cap) {
+    const int group = num_q_heads / num_kv_heads;
+    const int64_t nrb = ((int64_t)max_q_len * group + kTqPrefillStreamRows - 1) / kTqPrefillStreamRows;
+    const double tokens = (double)num_seqs * num_kv_heads * nrb * (cap + 4.0 * kTqPrefillStreamRows);
+    const double w = tokens / 128 + 1;
+    return w < kStreamWorkers ? (int64_t)w : kStreamWorkers;
+}
+size_t stream_bytes(int64_t workers) {
+    return (size_t)workers * (2 * kTqPrefillStreamRows * (TQ_HEAD_DIM + 2) * sizeof(float) + sizeof(TqPrefillCut));
+}
+
+// prefill_stream_kernel reads lane-grouped tiles whose norms follow their payload within 2 GiB at its
+// strides, 8-byte aligned; q is the QJL operand too; rows of q and out take vector accesses; the
+// scores' scale is positive (it compares them unscaled).
+bool stream_ok(const tq_kv_view* k, const tq_kv_view* v, const void* q_proj) {
+    if (k->layout != TQ_TILE_KEYS || v->layout != TQ_TILE_VALUES || (q_proj && k->qjl)) return false;
+    auto with = [](const tq_region& pay, const tq_region& nrm) {
+        const int64_t d = static_cast<const uint8_t*>(nrm.ptr) - static_cast<const uint8_t*>(pay.ptr);
+        return nrm.stride_row == 2 && nrm.stride_block == pay.stride_block && nrm.stride_head == pay.stride_head &&
+               aligned(nrm.ptr, 8) && nrm.stride_block % 8 == 0 && nrm.stride_head % 8 == 0 && d >= 0 &&
+               d < (1ll << 31) && pay.stride_block > 0 && pay.stride_block < (1ll << 31);
+    };
+    return with(k->idx, k->norm) && with(v->idx, v->norm) && (!k->qjl || with(k->idx, k->rnorm));
+}
+
+int prefill_impl(const void* q, int q_dtype, int64_t q_stride_token, int64_t q_stride_head,
                           const void* q_proj, int64_t qp_stride_token, int64_t qp_stride_head,
                           const int32_t* cu_seqlens_q, int num_seqs, int max_q_len,
                           int num_q_heads, int num_kv_heads, int head_dim,
@@ -554,7 +607,7 @@ extern "C" int tq_prefill(const void* q, int q_dtype, int64_t q_stride_token, in
                           const int32_t* block_tables, int64_t block_table_stride, int max_blocks_per_seq,
                           const int32_t* seq_lens, float sm_scale, float corr_scale, int flags,
                           void* out, int out_dtype, int64_t out_stride_token, int64_t out_stride_head,
-                          tq_stream_t stream) {
+                          void* workspace, size_t workspace_bytes, tq_stream_t stream) {
     if (head_dim != TQ_HEAD_DIM) return TQ_ERR_HEAD_DIM;
     if (!k || !v) return TQ_ERR_INVALID_ARGUMENT;
     if (num_seqs < 0 || max_q_len < 0 || num_q_heads <= 0 || num_kv_heads <= 0) return TQ_ERR_INVALID_ARGUMENT;
@@ -594,6 +647,65 @@ extern "C" int tq_prefill(const void* q, int q_dtype, int64_t q_stride_token, in
     const int64_t n_rb = (rows + kRowsPerWG - 1) / kRowsPerWG;
     const int64_t grid = n_rb * num_seqs * num_kv_heads;
     if (grid > 0x7fffffff) return TQ_ERR_INVALID_ARGUMENT;
+
+    const int64_t cap = (int64_t)max_blocks_per_seq * block_size;
+    if (cap > kStreamMinTokens && sm_scale > 1e-30f && stream_ok(k, v, q_proj) && rows < (1ll << 31) - 64 &&
+        q_vector_ok(q, q_dtype, q_stride_token, q_stride_head) && q_vector_ok(out, out_dtype, out_stride_token, out_stride_head)) {
+        int cus = 0;
+        if ((rc = device_cus(&cus))) return rc;
+        int64_t workers = stream_workers(num_seqs, max_q_len, num_q_heads, num_kv_heads, cap);
+        if (workers > (int64_t)cus * kTqPrefillStreamWaves) workers = (int64_t)cus * kTqPrefillStreamWaves;
+        TqPrefillStream t = {};
+        t.q = q;
+        t.q_st = q_stride_token;
+        t.q_sh = q_stride_head;
+        t.q_dtype = q_dtype;
+        t.cu_q = cu_seqlens_q;
+        t.num_seqs = num_seqs;
+        t.max_q = max_q_len;
+        t.hkv = num_kv_heads;
+        t.group = group;
+        auto bytes = [](const tq_region& r) { return static_cast<const uint8_t*>(r.ptr); };
+        t.kptr = bytes(k->idx);
+        t.d_kn = (uint32_t)(bytes(k->norm) - t.kptr);
+        t.d_kr = k->qjl ? (uint32_t)(bytes(k->rnorm) - t.kptr) : 0u;
+        t.vptr = bytes(v->idx);
+        t.d_vn = (uint32_t)(bytes(v->norm) - t.vptr);
+        t.k_sb = (uint32_t)k->idx.stride_block;
+        t.k_sh = k->idx.stride_head;
+        t.v_sb = (uint32_t)v->idx.stride_block;
+        t.v_sh = v->idx.stride_head;
+        t.k_cent = k->centroids;
+        t.v_cent = v->centroids;
+        t.k_cs = k->centroid_scale > 0.f ? k->centroid_scale : 1.f;
+        t.v_cs = v->centroid_scale > 0.f ? v->centroid_scale : 1.f;
+        t.v_cinv = 1.f / t.v_cs;
+        t.share = k->centroids == v->centroids && k->bits == v->bits && t.k_cs == t.v_cs;
+        t.block_size = block_size;
+        t.tpb = block_size / 16;
+        t.tpb_div = tq_make_udiv((uint32_t)t.tpb);
+        t.num_blocks = num_blocks < 0x7fffffff ? (uint32_t)num_blocks : 0x7fffffffu;
+        t.bt = block_tables;
+        t.bt_stride = block_table_stride;
+        t.max_blocks = max_blocks_per_seq;
+        t.seq_lens = seq_lens;
+        t.c1 = sm_scale * kLog2e / t.k_cs;
+        t.c2 = sm_scale * kLog2e * corr_scale;
+        t.causal = (flags & TQ_PREFILL_CAUSAL) ? 1 : 0;
+        t.rot = (flags & TQ_PREFILL_ROTATE) ? 1 : 0;
+        t.out = out;
+        t.out_dtype = out_dtype;
+        t.out_st = out_stride_token;
+        t.out_sh = out_stride_head;
+        t.n_workers = (int)workers;
+        t.snap = !workspace || !aligned(workspace, 256) || workspace_bytes < stream_bytes(workers);
+        if (!t.snap) {
+            t.ws_acc = static_cast<float*>(workspace);
+            t.ws_ml = t.ws_acc + workers * 2 * kTqPrefillStreamRows * TQ_HEAD_DIM;
+            t.plan = reinterpret_cast<TqPrefillCut*>(t.ws_ml + workers * 2 * kTqPrefillStreamRows * 2);
+        }
+        return tq_prefill_stream_launch(t, k->bits, k->qjl != 0, v->bits, cus, (hipStream_t)stream);
+    }
 
     PrefillParams p = {};
     p.q = q;
@@ -647,4 +759,49 @@ extern "C" int tq_prefill(const void* q, int q_dtype, int64_t q_stride_token, in
     if (le != hipSuccess) return (int)le;
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? TQ_OK : (int)e;
+}
+
+}  // namespace
+
+extern "C" int tq_prefill(const void* q, int q_dtype, int64_t q_stride_token, int64_t q_stride_head,
+                          const void* q_proj, int64_t qp_stride_token, int64_t qp_stride_head,
+                          const int32_t* cu_seqlens_q, int num_seqs, int max_q_len,
+                          int num_q_heads, int num_kv_heads, int head_dim,
+                          const tq_kv_view* k, const tq_kv_view* v,
+                          int block_size, int64_t num_blocks,
+                          const int32_t* block_tables, int64_t block_table_stride, int max_blocks_per_seq,
+                          const int32_t* seq_lens, float sm_scale, float corr_scale, int flags,
+                          void* out, int out_dtype, int64_t out_stride_token, int64_t out_stride_head,
+                          tq_stream_t stream) {
+    return prefill_impl(q, q_dtype, q_stride_token, q_stride_head, q_proj, qp_stride_token, qp_stride_head, cu_seqlens_q,
+                        num_seqs, max_q_len, num_q_heads, num_kv_heads, head_dim, k, v, block_size, num_blocks,
+                        block_tables, block_table_stride, max_blocks_per_seq, seq_lens, sm_scale, corr_scale, flags, out,
+                        out_dtype, out_stride_token, out_stride_head, nullptr, 0, stream);
+}
+
+extern "C" size_t tq_prefill_workspace_bytes(int num_seqs, int max_q_len, int num_q_heads, int num_kv_heads,
+                                             int max_blocks_per_seq, int block_size) {
+    if (num_seqs <= 0 || max_q_len <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || num_q_heads % num_kv_heads ||
+        max_blocks_per_seq < 0 || block_size <= 0)
+        return 0;
+    const int64_t cap = (int64_t)max_blocks_per_seq * block_size;
+    if (cap <= kStreamMinTokens) return 0;
+    return stream_bytes(stream_workers(num_seqs, max_q_len, num_q_heads, num_kv_heads, cap));
+}
+
+extern "C" int tq_prefill_split(const void* q, int q_dtype, int64_t q_stride_token, int64_t q_stride_head,
+                                const void* q_proj, int64_t qp_stride_token, int64_t qp_stride_head,
+                                const int32_t* cu_seqlens_q, int num_seqs, int max_q_len,
+                                int num_q_heads, int num_kv_heads, int head_dim,
+                                const tq_kv_view* k, const tq_kv_view* v,
+                                int block_size, int64_t num_blocks,
+                                const int32_t* block_tables, int64_t block_table_stride, int max_blocks_per_seq,
+                                const int32_t* seq_lens, float sm_scale, float corr_scale, int flags,
+                                void* workspace, size_t workspace_bytes,
+                                void* out, int out_dtype, int64_t out_stride_token, int64_t out_stride_head,
+                                tq_stream_t stream) {
+    return prefill_impl(q, q_dtype, q_stride_token, q_stride_head, q_proj, qp_stride_token, qp_stride_head, cu_seqlens_q,
+                        num_seqs, max_q_len, num_q_heads, num_kv_heads, head_dim, k, v, block_size, num_blocks,
+                        block_tables, block_table_stride, max_blocks_per_seq, seq_lens, sm_scale, corr_scale, flags, out,
+                        out_dtype, out_stride_token, out_stride_head, workspace, workspace_bytes, stream);
 }

@@ -134,6 +134,13 @@ SIGNATURES = {
          ctypes.POINTER(TQKVView), ctypes.POINTER(TQKVView), _i32, _i64, _vp, _i64, _i32, _vp,
          _f32, _f32, _i32, _vp, _i32, _i64, _i64, _vp],
     ),
+    "tq_prefill_split": (
+        _i32,
+        [_vp, _i32, _i64, _i64, _vp, _i64, _i64, _vp, _i32, _i32, _i32, _i32, _i32,
+         ctypes.POINTER(TQKVView), ctypes.POINTER(TQKVView), _i32, _i64, _vp, _i64, _i32, _vp,
+         _f32, _f32, _i32, _vp, _sz, _vp, _i32, _i64, _i64, _vp],
+    ),
+    "tq_prefill_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32, _i32, _i32]),
     "tq_decode_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32]),
     "tq_decode_sparse_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32, _i32]),
     "tq_decode_noalloc": (

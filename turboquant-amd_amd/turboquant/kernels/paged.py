@@ -721,7 +721,14 @@ def prefill_paged(
     vv = paged_view(v_cache, v_fmt, vc)
     flags = (PREFILL_CAUSAL if causal else 0) | (PREFILL_ROTATE if rotate else 0)
     mq = T if max_q_len is None else int(max_q_len)
-    rc = _lib.lib().tq_prefill(
+    L = _lib.lib()
+    # (a buffer of this call: of the current stream, and of the graph under capture)
+    nws = L.tq_prefill_workspace_bytes(S, mq, Hq, Hkv, block_tables.shape[1], k_fmt.block_size)
+    try:
+        ws = torch.empty(nws, dtype=torch.uint8, device=dev) if nws else None
+    except torch.OutOfMemoryError:
+        ws, nws = None, 0
+    rc = L.tq_prefill_split(
         q.data_ptr(), _lib.dtype_code(q), q.stride(0), q.stride(1),
         _lib.ptr(q_proj), q_proj.stride(0) if q_proj is not None else 0, q_proj.stride(1) if q_proj is not None else 0,
         cu_seqlens_q.data_ptr(), S, mq, Hq, Hkv, 128,
@@ -729,9 +736,9 @@ def prefill_paged(
         block_tables.data_ptr(), block_tables.stride(0), block_tables.shape[1], seq_lens.data_ptr(),
         float((1.0 / math.sqrt(128)) if sm_scale is None else sm_scale),
         float((math.sqrt(math.pi / 2) / 128) if corr_scale is None else corr_scale), flags,
-        out.data_ptr(), _lib.dtype_code(out), out.stride(0), out.stride(1), _lib.stream_handle(dev),
+        _lib.ptr(ws), nws, out.data_ptr(), _lib.dtype_code(out), out.stride(0), out.stride(1), _lib.stream_handle(dev),
     )
-    _lib.check(rc, "tq_prefill")
+    _lib.check(rc, "tq_prefill_split")
     return out
 
 
