@@ -230,6 +230,20 @@ def test_decode_balanced_many_sequences(dev, kb, kq, vb, G, bs, scale):
     assert np.all(got[np.array(lens) == 0] == 0.0)
 
 
+@pytest.mark.parametrize("lens,Hkv", [([500], 1), ([540, 40], 2), ([1025], 1), ([1500], 2), ([2049], 1), ([4090, 0, 64], 2),
+                                      ([4097], 1), ([9000, 300], 2)])
+def test_decode_balanced_merge_waves(dev, lens, Hkv):
+    """Few long sequences under the balanced schedule: one pair per wave, so 16 to 282 pieces per segment,
+    merged by 1, 2, 4, 8 or 16 waves (both sides of each step), short and empty sequences beside them."""
+    Hq = 4 * Hkv
+    case = build_case(len(lens) + lens[0], len(lens), Hq, Hkv, lens, 4, False, 4, 16)
+    sm = 1 / math.sqrt(128)
+    got, _, qr = run_gpu(dev, case, Hq, Hkv, 4, False, 4, 16, sm, 0.0, chunk=0)
+    want, _, _ = oracle_out(case, Hq, Hkv, 4, False, 4, sm, 0.0, q_round=qr)
+    np.testing.assert_allclose(got, want, rtol=RTOL, atol=ATOL)
+    assert np.all(got[np.array(lens) == 0] == 0.0)
+
+
 def test_decode_balanced_all_empty(dev):
     """No tokens at all: no wave has work, the plan still says so, every output is zero."""
     lens = [0, 0, 0]
