@@ -260,7 +260,7 @@ def centroid_scale(centroids: torch.Tensor) -> float:
     The decode kernels keep fp16 centroid tables; tabulating s * c and dividing s back out in
     fp32 makes the table nearly exact (3-bit: 1.8e-4 -> 1.8e-5).  Cached per tensor version, so a
     device-resident codebook is read back once."""
-    key = (centroids.data_ptr(), centroids._version, centroids.numel(), str(centroids.device))
+    key = (centroids.data_ptr(), centroids._version, centroids.numel(), centroids.get_device())
     hit = _scale_cache.get(key)
     if hit is not None:
         return hit
