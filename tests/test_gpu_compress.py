@@ -218,6 +218,24 @@ def test_compress_k_v_against_oracle(dev, bits, n, parity_log):
     np.testing.assert_array_equal(v_norm.cpu().numpy(), k_norm.cpu().numpy())
 
 
+@pytest.mark.parametrize("bits", [1, 2, 3, 4])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_compress_k_v_row_tiles_per_wave(dev, bits, dtype):
+    """One row tile per wave up to 32768 rows on 256 CUs, two above: the last size of one and the first of
+    the other, and an odd piece, give every row the same bytes (the sums run in the same order)."""
+    from turboquant.kernels.packed_compress import compress_k, compress_v
+    cut = 128 * torch.cuda.get_device_properties(dev).multi_processor_count
+    g = torch.Generator().manual_seed(bits)
+    X = torch.randn(cut + 1, 128, generator=g).to(dtype).to(dev)
+    PiT, PiST = (m.to(dev) for m in _random_rotation(5))
+    cent, bnd = (m.to(dev) for m in _kernel_codebook(bits))
+    whole = (*compress_k(X, PiT, PiST, cent, bnd), *compress_v(X, PiT, cent, bnd))
+    for n in (cut, 1001):
+        part = (*compress_k(X[:n], PiT, PiST, cent, bnd), *compress_v(X[:n], PiT, cent, bnd))
+        for w, q in zip(whole, part):
+            assert torch.equal(w[:n].view(torch.uint8), q.view(torch.uint8))
+
+
 def test_compress_k_v_input_dtypes_and_rejections(dev):
     from turboquant.kernels.packed_compress import compress_k, compress_v
     PiT, PiST = _random_rotation(5)

@@ -52,7 +52,15 @@ template <bool PROJ>
 constexpr int packed_wg_waves() {
     return PROJ ? 8 : 4;
 }
-constexpr int kRT = 2;            // 16-row tiles per wave and pass
+// Rows per wave and pass: two 16-row tiles share every matrix fragment read from LDS; one tile, its loops
+// rolled (the code runs once, from a cold instruction cache) and its rows requested before the matrices are
+// staged, while the resident waves take all rows in one pass (n_rows <= 32768 on 256 CUs).  2-bit keys, fp32:
+// 1024 rows 44.1 -> 17.6 us, 32768 rows 45.9 -> 20.4 (26.4 with two tiles); above, two tiles 65536 rows
+// 48.2 -> 30.2 (31.7 rolled), 524288 rows 262 -> 170 (184 rolled).  Most of it is the matrices' alignment
+// in LDS: behind the static arrays they began 4 bytes off a multiple of 16, and every fragment read ran
+// as an unaligned access (a product of 16 rows 17000 cycles; 3800 aligned).
+// Bound: staging of the matrices (a third of a small call), then LDS reads and the VALU of the
+// quantisation.
 constexpr float kNearRel = 1.0f / (1 << 19);  // band: kNearRel * max column norm + kNearAbs
 constexpr float kNearAbs = 1.0f / (1 << 21);
 
@@ -104,13 +112,15 @@ __host__ __device__ constexpr int perm2(int p) {
     return (p & 7) < 4 ? 4 * (p >> 3) + (p & 7) : 16 + 4 * (p >> 3) + (p & 7) - 4;
 }
 
-template <int BITS, bool PROJ, int DT>
+template <int BITS, bool PROJ, int DT, int kRT>
 __global__ __launch_bounds__(packed_wg_waves<PROJ>() * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void packed_compress_mfma_kernel(PackedParams p) {
     constexpr int kWaves = packed_wg_waves<PROJ>();
     constexpr int NC = 1 << BITS;
     constexpr int NB = NC - 1;
-    extern __shared__ _Float16 s_h[];
+    constexpr int kCB = kRT == 1 ? 2 : 1;
+    constexpr int kPassUnroll = kRT == 1 ? 1 : 2, kSliceUnroll = kRT == 1 ? 1 : 4;
+    extern __shared__ __attribute__((aligned(16))) _Float16 s_h[];
     _Float16* s_m1h = s_h;                      // PiT^T hi  [col][d]
     _Float16* s_m1l = s_h + kD * kStride;       // PiT^T lo
     _Float16* s_m2h = s_h + 2 * kD * kStride;   // PiST^T hi [col][32ks + p] = PiST[32ks + perm2(p)][col]
@@ -120,6 +130,35 @@ void packed_compress_mfma_kernel(PackedParams p) {
     __shared__ float s_cent[NC];
 
     const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15;   // data row within the tile (B column / output column)
+    const int g = lane >> 4;   // K group of the operands; output rows 4g..4g+3 of a column block
+
+    const int64_t rows_per_pass = 16 * kRT;
+    const int64_t ngroups = (p.n_rows + rows_per_pass - 1) / rows_per_pass;
+    // rows of group grp: 32 elements of row n of each tile.  With one tile the first are on their way while
+    // the matrices are staged (two leave no registers for that)
+    float xv[kRT][4][8];
+    auto load_x = [&](int64_t grp) {
+#pragma unroll
+        for (int rt = 0; rt < kRT; ++rt) {
+            const int64_t row = grp * rows_per_pass + 16 * rt + n;
+            const bool live = grp < ngroups && row < p.n_rows;
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                const int64_t off = row * p.x_stride + 32 * ks + 8 * g;
+                if (live && p.x_vec) {
+                    tq_load8(p.x, off, DT, xv[rt][ks]);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) xv[rt][ks][e] = live ? tq_load1(p.x, off + e, DT) : 0.f;
+                }
+            }
+        }
+    };
+    const int64_t grp0 = (int64_t)blockIdx.x * kWaves + wave, grp_step = (int64_t)gridDim.x * kWaves;
+    if (kRT == 1) load_x(grp0);
     // float4 of 4 consecutive columns per thread and step (kWaves * 64 * 4 is a multiple of 128:
     // each thread keeps the same 4 columns and sums their squares)
     // Staging: task t = (column col = t % 128, group j = t / 128 of 8 positions along d) reads
@@ -129,7 +168,7 @@ void packed_compress_mfma_kernel(PackedParams p) {
     constexpr int kThreads = kWaves * 64;
     constexpr int kTasks = kD * (kD / 8) / kThreads;
     float css = 0.f;
-#pragma unroll
+#pragma unroll 1
     for (int k = 0; k < kTasks; ++k) {
         const int t = tid + k * kThreads;
         const int col = t & (kD - 1), j = t >> 7;
@@ -197,40 +236,21 @@ void packed_compress_mfma_kernel(PackedParams p) {
         near = m - near_thr;
     };
 
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int n = lane & 15;   // data row within the tile (B column / output column)
-    const int g = lane >> 4;   // K group of the operands; output rows 4g..4g+3 of a column block
-
-    const int64_t rows_per_pass = 16 * kRT;
-    const int64_t ngroups = (p.n_rows + rows_per_pass - 1) / rows_per_pass;
-    for (int64_t grp = (int64_t)blockIdx.x * kWaves + wave; grp < ngroups; grp += (int64_t)gridDim.x * kWaves) {
+    for (int64_t grp = grp0; grp < ngroups; grp += grp_step) {
+        if (kRT != 1) load_x(grp);
         const int64_t row0 = grp * rows_per_pass;
         // ---- rows: load, fp64 norm, x_n, fp16 hi / lo B operands ----
         tq_half8 bh[kRT][4], bl[kRT][4];
         float norm32[kRT];
 #pragma unroll
         for (int rt = 0; rt < kRT; ++rt) {
-            const int64_t row = row0 + 16 * rt + n;
-            const bool live = row < p.n_rows;
-            float xv[4][8];
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) {
-                const int64_t off = row * p.x_stride + 32 * ks + 8 * g;
-                if (live && p.x_vec) {
-                    tq_load8(p.x, off, DT, xv[ks]);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) xv[ks][e] = live ? tq_load1(p.x, off + e, DT) : 0.f;
-                }
-            }
             // fp64 norm, x_n rounded once from x * (1 / (norm + 1e-8)): an error in the norm
             // would scale rot, whose projection rot @ PiST is much larger than the residual's
             double ss = 0.0;
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-                for (int e = 0; e < 8; ++e) ss = __builtin_fma((double)xv[ks][e], (double)xv[ks][e], ss);
+                for (int e = 0; e < 8; ++e) ss = __builtin_fma((double)xv[rt][ks][e], (double)xv[rt][ks][e], ss);
             ss += __shfl_xor(ss, 16, 64);
             ss += __shfl_xor(ss, 32, 64);
             const double nrm = __builtin_sqrt(ss);
@@ -247,7 +267,7 @@ void packed_compress_mfma_kernel(PackedParams p) {
                     // x_n rounded to fp32 first (the hi part is then one fp32 -> fp16 conversion;
                     // left to itself the compiler turns fp64 -> fp32 -> fp16 into a software
                     // fp64 -> fp16 rounding of ~25 instructions per element)
-                    float xn = (float)((double)xv[ks][e] * inv);
+                    float xn = (float)((double)xv[rt][ks][e] * inv);
                     asm("" : "+v"(xn));
                     const _Float16 h = (_Float16)xn;
                     bh[rt][ks][e] = h;
@@ -255,37 +275,64 @@ void packed_compress_mfma_kernel(PackedParams p) {
                 }
         }
 
-        // ---- rot^T = PiT^T x_n^T ----
-        // 32 steps (K slice ks = step / 8, column block cb = step % 8); the A fragments of the
-        // next step are loaded before this step's products (the barrier keeps the schedule to
-        // that one step of look-ahead: hoisting all 64 loads runs out of registers)
+        if (kRT == 1 && grp + grp_step < ngroups) load_x(grp + grp_step);
+
         tq_floatx4 acc[kRT][8];
+        uint32_t rnorm16[kRT];  // fp16 bits, rounded once from the product
+#pragma unroll kPassUnroll
+        for (int pass = 0; pass < (PROJ ? 2 : 1); ++pass) {
+        // ---- pass 0: rot^T = PiT^T x_n^T; pass 1: proj^T = PiST^T resid^T ----
+        // K slices in turn (the operands moved up after each), steps of kCB column blocks (with one row
+        // tile two, so that a step has independent products); the A fragments of the next step are
+        // loaded before this step's products (the barrier keeps the schedule to that one step of
+        // look-ahead).
 #pragma unroll
         for (int rt = 0; rt < kRT; ++rt)
 #pragma unroll
             for (int cb = 0; cb < 8; ++cb) acc[rt][cb] = tq_floatx4{0.f, 0.f, 0.f, 0.f};
         {
-            tq_half8 ah[2], al[2];
-            auto frag = [&](int step, tq_half8& h, tq_half8& l) {
-                const int o = (16 * (step & 7) + n) * kStride + 32 * (step >> 3) + 8 * g;
-                h = *reinterpret_cast<const tq_half8*>(s_m1h + o);
-                l = *reinterpret_cast<const tq_half8*>(s_m1l + o);
-            };
-            frag(0, ah[0], al[0]);
+            const _Float16* mh = s_m1h + pass * (2 * kD * kStride) + n * kStride + 8 * g;
+            tq_half8 ah[2][kCB], al[2][kCB];
+            auto frag = [&](const _Float16* m, int cb, tq_half8 (&h)[kCB], tq_half8 (&l)[kCB]) {
 #pragma unroll
-            for (int step = 0; step < 32; ++step) {
-                if (step + 1 < 32) frag(step + 1, ah[(step + 1) & 1], al[(step + 1) & 1]);
-                const int ks = step >> 3, cb = step & 7;
-#pragma unroll
-                for (int rt = 0; rt < kRT; ++rt) {
-                    acc[rt][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[step & 1], bh[rt][ks], acc[rt][cb], 0, 0, 0);
-                    acc[rt][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[step & 1], bl[rt][ks], acc[rt][cb], 0, 0, 0);
-                    acc[rt][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[step & 1], bh[rt][ks], acc[rt][cb], 0, 0, 0);
+                for (int c = 0; c < kCB; ++c) {
+                    h[c] = *reinterpret_cast<const tq_half8*>(m + 16 * (cb + c) * kStride);
+                    l[c] = *reinterpret_cast<const tq_half8*>(m + 16 * (cb + c) * kStride + kD * kStride);
                 }
-                __builtin_amdgcn_sched_barrier(0);
+            };
+            frag(mh, 0, ah[0], al[0]);
+#pragma unroll kSliceUnroll
+            for (int ks = 0; ks < 4; ++ks) {
+                const _Float16* next = mh + (ks < 3 ? 32 : 0);
+#pragma unroll
+                for (int step = 0; step < 8 / kCB; ++step) {
+                    const int cb = kCB * step;
+                    if (cb + kCB < 8) frag(mh, cb + kCB, ah[(step + 1) & 1], al[(step + 1) & 1]);
+                    else frag(next, 0, ah[(step + 1) & 1], al[(step + 1) & 1]);
+                    // hi hi, hi lo, lo hi of each sum, the sums in turn
+#pragma unroll
+                    for (int part = 0; part < 3; ++part)
+#pragma unroll
+                        for (int i = 0; i < kRT * kCB; ++i) {
+                            const int rt = i / kCB, c = i % kCB;
+                            acc[rt][cb + c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(part < 2 ? ah[step & 1][c] : al[step & 1][c],
+                                                                                     part == 1 ? bl[rt][0] : bh[rt][0],
+                                                                                     acc[rt][cb + c], 0, 0, 0);
+                        }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                mh = next;
+#pragma unroll
+                for (int rt = 0; rt < kRT; ++rt)
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) {
+                        bh[rt][k] = bh[rt][k + 1];
+                        bl[rt][k] = bl[rt][k + 1];
+                    }
             }
         }
 
+        if (pass == 0) {
         // ---- indices (BITS-bit fields of the 4 elements of (rt, cb), word 8 rt + cb) and the
         // elements near a boundary.  Element e = 32 rt + 4 cb + r of a lane is
         // rot[row0 + 16 rt + n][16 cb + 4 g + r]. ----
@@ -343,8 +390,6 @@ void packed_compress_mfma_kernel(PackedParams p) {
         }
 
         // ---- indices, residuals, packing ----
-        tq_half8 rh[kRT][4], rl[kRT][4];
-        float rnorm[kRT];
 #pragma unroll
         for (int rt = 0; rt < kRT; ++rt) {
             const int64_t row = row0 + 16 * rt + n;
@@ -363,8 +408,8 @@ void packed_compress_mfma_kernel(PackedParams p) {
                         rss = __builtin_fmaf(rs, rs, rss);
                         // B operand of the second product: slice cb / 2, position 8g + 4 (cb & 1) + r
                         const _Float16 h = (_Float16)rs;
-                        rh[rt][cb >> 1][4 * (cb & 1) + r] = h;
-                        rl[rt][cb >> 1][4 * (cb & 1) + r] = (_Float16)(rs - (float)h);
+                        bh[rt][cb >> 1][4 * (cb & 1) + r] = h;
+                        bl[rt][cb >> 1][4 * (cb & 1) + r] = (_Float16)(rs - (float)h);
                     }
                 }
                 // this lane's 4 fields sit at bit 4 g BITS of the column block's 16-field segment
@@ -372,7 +417,7 @@ void packed_compress_mfma_kernel(PackedParams p) {
                 seg[cb][0] = or_over_groups((uint32_t)f);
                 if (BITS > 2) seg[cb][BITS > 2 ? 1 : 0] = or_over_groups((uint32_t)(f >> 32));
             }
-            if (PROJ) rnorm[rt] = __builtin_sqrtf(sum_over_groups(rss)) * norm32[rt];
+            if (PROJ) rnorm16[rt] = tq_f32_to_f16_bits(__builtin_sqrtf(sum_over_groups(rss)) * norm32[rt]);
             if (row < p.n_rows) {
                 // lane group g stores column blocks 2g and 2g + 1: 4 BITS bytes at byte 4 g BITS
                 uint32_t w[BITS];
@@ -406,34 +451,8 @@ void packed_compress_mfma_kernel(PackedParams p) {
             }
         }
 
-        if (PROJ) {
-            // ---- proj^T = PiST^T resid^T (resid without its factor norm > 0: same signs) ----
-            tq_floatx4 pj[kRT][8];
-#pragma unroll
-            for (int rt = 0; rt < kRT; ++rt)
-#pragma unroll
-                for (int cb = 0; cb < 8; ++cb) pj[rt][cb] = tq_floatx4{0.f, 0.f, 0.f, 0.f};
-            {
-                tq_half8 ah[2], al[2];
-                auto frag = [&](int step, tq_half8& h, tq_half8& l) {
-                    const int o = (16 * (step & 7) + n) * kStride + 32 * (step >> 3) + 8 * g;
-                    h = *reinterpret_cast<const tq_half8*>(s_m2h + o);
-                    l = *reinterpret_cast<const tq_half8*>(s_m2l + o);
-                };
-                frag(0, ah[0], al[0]);
-#pragma unroll
-                for (int step = 0; step < 32; ++step) {
-                    if (step + 1 < 32) frag(step + 1, ah[(step + 1) & 1], al[(step + 1) & 1]);
-                    const int ks = step >> 3, cb = step & 7;
-#pragma unroll
-                    for (int rt = 0; rt < kRT; ++rt) {
-                        pj[rt][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[step & 1], rh[rt][ks], pj[rt][cb], 0, 0, 0);
-                        pj[rt][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[step & 1], rl[rt][ks], pj[rt][cb], 0, 0, 0);
-                        pj[rt][cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[step & 1], rh[rt][ks], pj[rt][cb], 0, 0, 0);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
+        } else {
+            // ---- signs (resid went without its factor norm > 0: same signs) ----
 #pragma unroll
             for (int rt = 0; rt < kRT; ++rt) {
                 const int64_t row = row0 + 16 * rt + n;
@@ -443,15 +462,16 @@ void packed_compress_mfma_kernel(PackedParams p) {
                 for (int cb = 0; cb < 8; ++cb) {
                     uint32_t f = 0;
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) f |= ((__float_as_uint(pj[rt][cb][r]) >> 31) ^ 1u) << r;
+                    for (int r = 0; r < 4; ++r) f |= ((__float_as_uint(acc[rt][cb][r]) >> 31) ^ 1u) << r;
                     f = zero ? 0xfu : f;
                     seg[cb] = or_over_groups(f << (4 * g));
                 }
                 if (row < p.n_rows) {
                     reinterpret_cast<uint32_t*>(p.signs_out + row * 16)[g] = pick_group(seg, g, 0) | (pick_group(seg, g, 1) << 16);
-                    if (g == 0) p.rnorm_out[row] = (uint16_t)tq_f32_to_f16_bits(rnorm[rt]);
+                    if (g == 0) p.rnorm_out[row] = (uint16_t)rnorm16[rt];
                 }
             }
+        }
         }
     }
 }
@@ -480,8 +500,18 @@ int tq_packed_mfma_launch(const void* x, int x_dtype, int64_t x_stride, int64_t 
     p.rnorm_out = rnorm_out;
     p.norm_out = norm_out;
     const bool proj = pist != nullptr;
+    int dev = 0, max_lds = 0, cus = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e != hipSuccess) return (int)e;
+    const int waves = proj ? packed_wg_waves<true>() : packed_wg_waves<false>();
+    const int64_t cap = (int64_t)cus * (proj ? 1 : 2);  // resident workgroups (LDS-limited)
+    const int rt = n_rows <= 16 * waves * cap ? 1 : 2;
     const void* kern = nullptr;
-#define TQ_PK_DT(B, PJ, DT) kern = (const void*)packed_compress_mfma_kernel<B, PJ, DT>
+#define TQ_PK_DT(B, PJ, DT)                                                               \
+    kern = rt == 1 ? (const void*)packed_compress_mfma_kernel<B, PJ, DT, 1> \
+                   : (const void*)packed_compress_mfma_kernel<B, PJ, DT, 2>
 #define TQ_PK(B, PJ)                                                \
     if (bits == B && proj == PJ) {                                  \
         if (x_dtype == TQ_BF16) TQ_PK_DT(B, PJ, TQ_BF16);           \
@@ -494,11 +524,6 @@ int tq_packed_mfma_launch(const void* x, int x_dtype, int64_t x_stride, int64_t 
 #undef TQ_PK_DT
     if (!kern) return TQ_ERR_BITS;
     const size_t lds = tq_packed_mfma_lds_bytes(proj);
-    int dev = 0, max_lds = 0, cus = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e == hipSuccess) e = hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
-    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e != hipSuccess) return (int)e;
     // the matrices (dynamic LDS) and the kernel's own arrays (static LDS) must fit
     hipFuncAttributes fa{};
     e = hipFuncGetAttributes(&fa, kern);
@@ -515,10 +540,8 @@ int tq_packed_mfma_launch(const void* x, int x_dtype, int64_t x_stride, int64_t 
             done.insert({kern, dev});
         }
     }
-    const int waves = proj ? packed_wg_waves<true>() : packed_wg_waves<false>();
-    const int64_t groups = (n_rows + 16 * kRT - 1) / (16 * kRT);
+    const int64_t groups = (n_rows + 16 * rt - 1) / (16 * rt);
     int64_t grid = (groups + waves - 1) / waves;
-    const int64_t cap = (int64_t)cus * (proj ? 1 : 2);  // resident workgroups (LDS-limited)
     grid = grid < cap ? grid : cap;
     void* args[] = {&p};
     e = hipLaunchKernel(kern, dim3((unsigned)grid), dim3(waves * 64), args, lds, st);
