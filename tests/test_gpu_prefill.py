@@ -225,3 +225,20 @@ def test_prefill_stream_shares(dev, monkeypatch, name, workspace, causal):
         monkeypatch.setattr(_lib.lib(), "tq_prefill_workspace_bytes", lambda *a: 0)
     got, _, _ = run_prefill(dev, case, q, cu, kb, kq, vb, bs, SM, CS, causal=causal, out_dtype=torch.float32)
     np.testing.assert_allclose(got, want, rtol=2 * RTOL, atol=2 * ATOL)
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("lens", [[6000], [250]])
+def test_prefill_bad_query_rows_stay_visible(dev, lens, bad):
+    """A query row that is not finite gives NaN, also where its keys are cut over several waves (6000
+    tokens), and leaves every other row as it was.  The other rows may round anew (their exponent base
+    moves with a row of the same tile): both runs are within RTOL / ATOL of the oracle."""
+    kb, kq, vb, Hkv, G, bs = 3, True, 3, 2, 4, 16
+    case = build_case(11, 1, G * Hkv, Hkv, lens, kb, kq, vb, bs)
+    q, cu = make_queries(np.random.default_rng(3), [50], G * Hkv)
+    want, _, _ = run_prefill(dev, case, q, cu, kb, kq, vb, bs, SM, CS, out_dtype=torch.float32)
+    q[7, 2] = bad
+    got, _, _ = run_prefill(dev, case, q, cu, kb, kq, vb, bs, SM, CS, out_dtype=torch.float32)
+    assert np.isnan(got[7, 2]).all()
+    got[7, 2] = want[7, 2]
+    np.testing.assert_allclose(got, want, rtol=2 * RTOL, atol=2 * ATOL)
