@@ -584,16 +584,17 @@ size_t stream_bytes(int64_t workers) {
     return (size_t)workers * (2 * kTqPrefillStreamRows * (TQ_HEAD_DIM + 2) * sizeof(float) + sizeof(TqPrefillCut));
 }
 
-// prefill_stream_kernel reads lane-grouped tiles whose norms follow their payload within 2 GiB at its
-// strides, 8-byte aligned; q is the QJL operand too; rows of q and out take vector accesses; the
-// scores' scale is positive (it compares them unscaled).
-bool stream_ok(const tq_kv_view* k, const tq_kv_view* v, const void* q_proj) {
+// prefill_stream_kernel reads lane-grouped tiles whose norms follow their payload at its strides, 8-byte
+// aligned, all of a tile within the 2 GiB that a buffer descriptor spans; q is the QJL operand too; rows
+// of q and out take vector accesses; the scores' scale is positive (it compares them unscaled).
+bool stream_ok(const tq_kv_view* k, const tq_kv_view* v, const void* q_proj, int block_size) {
+    if (block_size > (1 << 20)) return false;  // (payload at most 84 MB, norms 2 MB)
     if (k->layout != TQ_TILE_KEYS || v->layout != TQ_TILE_VALUES || (q_proj && k->qjl)) return false;
     auto with = [](const tq_region& pay, const tq_region& nrm) {
         const int64_t d = static_cast<const uint8_t*>(nrm.ptr) - static_cast<const uint8_t*>(pay.ptr);
         return nrm.stride_row == 2 && nrm.stride_block == pay.stride_block && nrm.stride_head == pay.stride_head &&
                aligned(nrm.ptr, 8) && nrm.stride_block % 8 == 0 && nrm.stride_head % 8 == 0 && d >= 0 &&
-               d < (1ll << 31) && pay.stride_block > 0 && pay.stride_block < (1ll << 31);
+               d < (1ll << 31) - (1 << 22) && pay.stride_block > 0 && pay.stride_block < (1ll << 31);
     };
     return with(k->idx, k->norm) && with(v->idx, v->norm) && (!k->qjl || with(k->idx, k->rnorm));
 }
@@ -649,7 +650,7 @@ int prefill_impl(const void* q, int q_dtype, int64_t q_stride_token, int64_t q_s
     if (grid > 0x7fffffff) return TQ_ERR_INVALID_ARGUMENT;
 
     const int64_t cap = (int64_t)max_blocks_per_seq * block_size;
-    if (cap > kStreamMinTokens && sm_scale > 1e-30f && stream_ok(k, v, q_proj) && rows < (1ll << 31) - 64 &&
+    if (cap > kStreamMinTokens && sm_scale > 1e-30f && stream_ok(k, v, q_proj, block_size) && rows < (1ll << 31) - 64 &&
         q_vector_ok(q, q_dtype, q_stride_token, q_stride_head) && q_vector_ok(out, out_dtype, out_stride_token, out_stride_head)) {
         int cus = 0;
         if ((rc = device_cus(&cus))) return rc;
