@@ -738,7 +738,7 @@ def main():
     if mfma is not None:
         details["mfma_busy_fraction_headline"] = mfma
     for name, prof in (("config3", "decode_fast_kernel_config3_pmc.md"), ("config5", "decode_fast_kernel_config5_pmc.md"),
-                       ("prefill", "prefill_kernel_4x4096_pmc.md")):
+                       ("prefill", "prefill_stream_kernel_4x4096.md")):
         v = profile_value(prof, "mfma_busy_fraction")
         if v is not None:
             details.setdefault("mfma_busy_fraction_by_kernel", {})[name] = v
