@@ -571,3 +571,12 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setenv("TQ_HIP_LIB", str(tmp_path / "nope.so"))
     with pytest.raises(_lib.TurboQuantError, match="no CPU fallback"):
         _lib.lib()
+
+
+def test_only_the_fast_decode_kernel_is_compiled_without_nan_semantics():
+    """The prefill kernels hand NaN scores of a query row on to its output; under -fno-honor-nans (or a
+    flag that implies it) a NaN operand is undefined, whatever one compiler makes of it."""
+    import build
+    nan_free = {"-fno-honor-nans", "-ffast-math", "-ffinite-math-only"}
+    assert not nan_free & set(build.COMMON_FLAGS)
+    assert [f for f, flags in build.FILE_FLAGS.items() if nan_free & set(flags)] == ["tq_decode_fast.hip"]

@@ -47,10 +47,11 @@ COMMON_FLAGS = [
 
 
 # Per-source flags.  The fast decode kernel never relies on NaN semantics (masked rows are
-# -inf, never NaN), so fmax needs no quieting of its operands.
+# -inf, never NaN), so fmax needs no quieting of its operands.  No other file may take the flag:
+# the prefill kernels hand a query row's NaN scores on to its output, and under the flag a NaN
+# operand is undefined.
 FILE_FLAGS = {
     "tq_decode_fast.hip": ["-fno-honor-nans"],
-    "tq_prefill_stream.hip": ["-fno-honor-nans"],
 }
 
 

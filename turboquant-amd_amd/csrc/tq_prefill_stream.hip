@@ -587,6 +587,19 @@ void prefill_stream_kernel(TqPrefillStream p) {
                             __builtin_amdgcn_sched_barrier(0);
                         }
                     }
+                    // The lane's largest score per row tile.  Worked out here, where the scores are products
+                    // fresh from the fused multiply-add: the compiler quiets the operands of a maximum that
+                    // come from another basic block, one more instruction each (24 a step: 4-bit, 4 x 4096
+                    // tokens 1343 -> 1380 us; here 1348).  With 2- and 4-bit keys with QJL, which spill more,
+                    // the quieting is cheaper (1612 -> 1651 us; here 1686).
+                    constexpr bool kEarlyMax = !KQJL || KB == 3;
+                    float mx[kRT];
+                    auto lane_max = [&](int rt) {
+                        return fmaxf(fmaxf(fmaxf(sv[rt][0], sv[rt][1]), fmaxf(sv[rt][2], sv[rt][3])),
+                                     fmaxf(fmaxf(sv[rt][4], sv[rt][5]), fmaxf(sv[rt][6], sv[rt][7])));
+                    };
+#pragma unroll
+                    for (int rt = 0; rt < kRT; ++rt) mx[rt] = kEarlyMax ? lane_max(rt) : 0.f;
                     // the next step's keys (the current ones are used up)
                     Where nxt = cur;
                     if (j + 1 < j1) {
@@ -606,6 +619,7 @@ void prefill_stream_kernel(TqPrefillStream p) {
                                 const int tok = (r & 3) + 16 * (r >> 2);
                                 sv[rt][r] = tok < lim && 4 * g + (r & 3) < cur.nv[r >> 2] ? sv[rt][r] : kNegInf;
                             }
+                            mx[rt] = lane_max(rt);
                         }
 #pragma unroll
                         for (int h = 0; h < 2; ++h)
@@ -625,8 +639,7 @@ void prefill_stream_kernel(TqPrefillStream p) {
                     tq_half8 bop[kRT];
 #pragma unroll
                     for (int rt = 0; rt < kRT; ++rt) {
-                        float mt = fmaxf(fmaxf(fmaxf(sv[rt][0], sv[rt][1]), fmaxf(sv[rt][2], sv[rt][3])),
-                                         fmaxf(fmaxf(sv[rt][4], sv[rt][5]), fmaxf(sv[rt][6], sv[rt][7])));
+                        float mt = kEarlyMax ? mx[rt] : lane_max(rt);
                         // M moves only when some row's score passes it, and then kHeadroom above the largest:
                         // p = exp2(c1 s - M) <= 1, and acc and lsum carry the same factor
                         if (__builtin_amdgcn_ballot_w64(__builtin_fmaf(mt, p.c1, -M[rt]) > 0.f)) {
