@@ -563,16 +563,19 @@ def test_sparse_v_reference_slot_layout(dev):
     assert abs(gsk - skipped) <= allow
 
 
+@pytest.mark.parametrize("chunk", [2080, 65536])
 @pytest.mark.parametrize("kb,qjl,vb,G,bs", [(3, False, 3, 6, 32), (2, True, 2, 4, 16), (3, True, 3, 12, 64), (4, False, 3, 8, 16)])
-def test_sparse_v_split_single_pass(dev, kb, qjl, vb, G, bs):
+def test_sparse_v_split_single_pass(dev, kb, qjl, vb, G, bs, chunk):
     """A single pass over several units per (sequence, KV head) (its maxima from a first pass over the
     keys) skips exactly the tokens that one unit per (sequence, KV head) skips, for lengths of nothing,
-    of less than a tile, of one unit and ends inside a unit, and past max_seq_len; the outputs differ
-    by the order of the fp32 sums (each probability is rounded to fp16 against the same running max)."""
+    of less than a tile, of one unit and ends inside a unit, and past max_seq_len (by more than a unit
+    where the chunk allows it); the outputs differ by the order of the fp32 sums (each probability is
+    rounded to fp16 against the same running max).  tq_decode_sparse_workspace_bytes is enough for the
+    split at any tokens_per_chunk, and the stream's own buffer runs the same."""
     from turboquant import _lib
     from turboquant.kernels.paged import PagedKVFormat, allocate_cache, compress_paged, decode_paged
     Hkv = 2
-    lens = [0, 5, 64, 1000, 1504, 2061]
+    lens = [0, 5, 64, 1000, 1504, 2061 if chunk < 3000 else 3001]
     S, Hq, msl = len(lens), Hkv * G, 2050
     g = torch.Generator(device=dev).manual_seed(kb)
     maxb = -(-max(lens) // bs)
@@ -587,17 +590,20 @@ def test_sparse_v_split_single_pass(dev, kb, qjl, vb, G, bs):
     compress_paged(torch.randn(n, Hkv, 128, generator=g, device=dev), slots, vc, vf, *vcb)
     bt = torch.randperm(S * maxb, generator=g, device=dev).to(torch.int32).view(S, maxb)
     q = torch.randn(S, Hq, 128, generator=g, device=dev) * 3
-    chunk = 2080
     got = []
     small = _lib.lib().tq_decode_workspace_bytes(S, Hq, msl, chunk)
-    assert _lib.lib().tq_decode_sparse_workspace_bytes(S, Hq, Hkv, msl, chunk) > small
-    for ws in (torch.empty(small, dtype=torch.uint8, device=dev), None):
+    split = _lib.lib().tq_decode_sparse_workspace_bytes(S, Hq, Hkv, msl, chunk)
+    assert split > small
+    full = torch.full((split,), 0xa5, dtype=torch.uint8, device=dev)
+    for ws in (torch.empty(small, dtype=torch.uint8, device=dev), full, None):
         st = torch.zeros(2, dtype=torch.int64, device=dev)
         out = decode_paged(q, kc, kf, kcb[0], vc, vf, vcb[0], bt, torch.tensor(lens, dtype=torch.int32, device=dev),
                            sparse_threshold=1e-2, max_seq_len=msl, tokens_per_chunk=chunk, workspace=ws, skip_stats=st)
         got.append((out, st.tolist()))
-    assert got[0][1] == got[1][1] and 0 < got[0][1][0] < got[0][1][1]
+    assert bool((full[small:] != 0xa5).any())  # several units ran
+    assert got[0][1] == got[1][1] == got[2][1] and 0 < got[0][1][0] < got[0][1][1]
     torch.testing.assert_close(got[1][0], got[0][0], rtol=1e-5, atol=1e-5)
+    assert torch.equal(got[2][0], got[1][0])
 
 
 @pytest.mark.parametrize("bs", [16, 32])

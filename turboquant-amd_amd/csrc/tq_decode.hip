@@ -499,7 +499,8 @@ void decode_kernel(DecodeParams p) {
     L = L < p.len_limit ? L : p.len_limit;
     const int t_begin = c * p.chunk;
     if (t_begin >= L) return;
-    const int t_end = (t_begin + p.chunk < L) ? t_begin + p.chunk : L;
+    // (the last chunk takes the rest: only a split single pass has more than a chunk there)
+    const int t_end = (c + 1 < p.n_chunks && t_begin + p.chunk < L) ? t_begin + p.chunk : L;
     const bool paged = p.bt != nullptr;
 
     // ---- query operands (B of the QK products), pre-scaled into the log2 domain ----
@@ -1380,15 +1381,14 @@ int tq_decode_impl(int rotate, const void* q, int q_dtype, int64_t q_stride_seq,
     if (!fast && !contig && n_chunks == 1 && sparse_threshold > 0.f && max_seq_len > 0 &&
         workspace_bytes >= tq_decode_sparse_workspace_bytes(num_seqs, num_q_heads, num_kv_heads, max_seq_len,
                                                             tokens_per_chunk)) {
-        // (units past max_seq_len, for sequences longer than it that the single pass would still
-        // take up to len_limit, must fit too; otherwise it stays one pass)
+        // (of a sequence longer than max_seq_len the last unit takes all that the single pass would,
+        // up to len_limit)
         int chunk = 0;
         const int n = single_pass_split(num_seqs, num_kv_heads, max_seq_len, &chunk);
-        const int n_all = n > 1 ? (len_limit + chunk - 1) / chunk : 1;
-        if (n > 1 && split_bytes(num_seqs, num_q_heads, n_all) <= workspace_bytes) {
+        if (n > 1) {
             split = true;
             tokens_per_chunk = chunk;
-            n_chunks = n_all;
+            n_chunks = n;
         }
     }
 
@@ -1590,8 +1590,8 @@ int tq_decode_impl(int rotate, const void* q, int q_dtype, int64_t q_stride_seq,
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
 
-    return launch_reduce(ws_acc, ws_m, ws_l, num_seqs, num_q_heads, n_chunks, tokens_per_chunk, len_limit, seq_lens, max_seq_len, out, out_dtype, out_stride_seq, out_stride_head,
-                         rotate, st);
+    return launch_reduce(ws_acc, ws_m, ws_l, num_seqs, num_q_heads, n_chunks, tokens_per_chunk, len_limit, seq_lens,
+                         max_seq_len, out, out_dtype, out_stride_seq, out_stride_head, rotate, st);
 }
 
 extern "C" size_t tq_packed_attention_workspace_bytes(int bh, int sk, int tokens_per_chunk) {

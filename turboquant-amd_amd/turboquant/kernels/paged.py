@@ -533,7 +533,8 @@ def run_decode(
         if sparse_threshold > 0:
             # room for a split single pass (a caller's own workspace decides that by its size)
             need = L.tq_decode_sparse_workspace_bytes(S, Hq, num_kv_heads, max_seq_len, tokens_per_chunk)
-        workspace = decode_workspace(dev, need)
+        # (the stream's buffer may be larger: what the call does depends on the call alone)
+        workspace = decode_workspace(dev, need)[:need]
     if skip_stats is not None and (skip_stats.dtype != torch.int64 or skip_stats.numel() < 2 or not skip_stats.is_cuda):
         raise ValueError("skip_stats must be a device int64 tensor with 2 elements")
     bt_ptr = block_tables.data_ptr() if block_tables is not None else None
