@@ -116,6 +116,21 @@ def test_prefill_block_sizes_row_blocks_and_short_sequences(dev, bs):
     assert np.all(got[int(cu[1]):int(cu[1]) + 2] == 0.0)
 
 
+def test_prefill_more_new_tokens_than_max_q_len(dev):
+    """A sequence with more new tokens than max_q_len: the ones that are computed keep their positions
+    (the causal limit counts all of the sequence's new tokens)."""
+    kb, kq, vb, Hq, Hkv, bs = 4, False, 4, 8, 2, 16
+    lens, n_new, mq = [300, 250], [70, 30], 64
+    case = build_case(61, len(lens), Hq, Hkv, lens, kb, kq, vb, bs)
+    rng = np.random.default_rng(5)
+    q, cu = make_queries(rng, n_new, Hq)
+    got, qr, _ = run_prefill(dev, case, q, cu, kb, kq, vb, bs, SM, CS, max_q_len=mq)
+    want = oracle_prefill(case, qr, cu, Hq, Hkv, kb, kq, vb, SM, CS)
+    for s, n in enumerate(n_new):
+        rows = slice(int(cu[s]), int(cu[s]) + min(n, mq))
+        np.testing.assert_allclose(got[rows], want[rows], rtol=RTOL, atol=ATOL)
+
+
 def test_prefill_rotated_and_explicit_q_proj(dev):
     kb, kq, vb, Hq, Hkv, bs = 3, True, 3, 8, 2, 16
     lens = [200, 45]

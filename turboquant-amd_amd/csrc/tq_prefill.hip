@@ -650,7 +650,8 @@ int prefill_impl(const void* q, int q_dtype, int64_t q_stride_token, int64_t q_s
     if (grid > 0x7fffffff) return TQ_ERR_INVALID_ARGUMENT;
 
     const int64_t cap = (int64_t)max_blocks_per_seq * block_size;
-    if (cap > kStreamMinTokens && sm_scale > 1e-30f && stream_ok(k, v, q_proj, block_size) && rows < (1ll << 31) - 64 &&
+    const int64_t grid_q = (n_rb * kRowsPerWG + group - 1) / group;  // new tokens that prefill_kernel's grid takes
+    if (cap > kStreamMinTokens && sm_scale > 1e-30f && stream_ok(k, v, q_proj, block_size) && grid_q * group < (1ll << 31) - 64 &&
         q_vector_ok(q, q_dtype, q_stride_token, q_stride_head) && q_vector_ok(out, out_dtype, out_stride_token, out_stride_head)) {
         int cus = 0;
         if ((rc = device_cus(&cus))) return rc;
@@ -663,7 +664,7 @@ int prefill_impl(const void* q, int q_dtype, int64_t q_stride_token, int64_t q_s
         t.q_dtype = q_dtype;
         t.cu_q = cu_seqlens_q;
         t.num_seqs = num_seqs;
-        t.max_q = max_q_len;
+        t.max_q = (int)grid_q;
         t.hkv = num_kv_heads;
         t.group = group;
         auto bytes = [](const tq_region& r) { return static_cast<const uint8_t*>(r.ptr); };

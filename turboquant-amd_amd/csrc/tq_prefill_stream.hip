@@ -172,14 +172,14 @@ struct Seq {
 __device__ __forceinline__ Seq seq_of(const TqPrefillStream& p, int s, bool whole) {
     Seq q;
     q.q0 = p.cu_q[s];
-    int nq = p.cu_q[s + 1] - q.q0;
-    nq = nq < p.max_q ? nq : p.max_q;
+    const int nq = p.cu_q[s + 1] - q.q0;
     q.nq = nq > 0 ? nq : 0;
+    const int computed = q.nq < p.max_q ? q.nq : p.max_q;  // (positions count all new tokens)
     int L = p.seq_lens[s];
     const int cap = p.max_blocks * p.block_size;
     L = L < cap ? L : cap;
     q.L = L > 0 ? L : 0;
-    q.nrb = (int)(((uint32_t)q.nq * (uint32_t)p.group + kRows - 1) / kRows);
+    q.nrb = (int)(((uint32_t)computed * (uint32_t)p.group + kRows - 1) / kRows);
     const int past = q.L > q.nq ? q.L - q.nq : 0;
     q.a = whole ? kMinTokens : (p.causal ? past + p.grow : q.L) + kSegTokens;
     q.step = whole ? 0 : p.step;
