@@ -257,3 +257,34 @@ def test_prefill_bad_query_rows_stay_visible(dev, lens, bad):
     assert np.isnan(got[7, 2]).all()
     got[7, 2] = want[7, 2]
     np.testing.assert_allclose(got, want, rtol=2 * RTOL, atol=2 * ATOL)
+
+
+@pytest.mark.parametrize("variant", ["rows", "q_proj", "unaligned_q", "unaligned_out", "zero_scale", "streams"])
+def test_prefill_takes_a_workspace_only_where_it_is_used(dev, variant):
+    """Calls that prefill_kernel serves allocate nothing beside their output; the streaming kernel's
+    allocate what tq_prefill_workspace_bytes says (here more than 32 MB)."""
+    from turboquant import _lib
+    from turboquant.kernels.paged import PagedKVFormat, allocate_cache, prefill_paged
+    S, n, Hq, Hkv, bs = 4, 256, 32, 8, 16
+    layouts = ("rows", "rows") if variant == "rows" else ("keys", "values")
+    kf = PagedKVFormat(bits=3, qjl=True, block_size=bs, layout=layouts[0])
+    vf = PagedKVFormat(bits=3, block_size=bs, layout=layouts[1])
+    nb = S * n // bs
+    kc, vc = allocate_cache(nb, Hkv, kf, device=dev).zero_(), allocate_cache(nb, Hkv, vf, device=dev).zero_()
+    bt = torch.arange(nb, dtype=torch.int32, device=dev).view(S, -1).repeat(1, 2)
+    lens = torch.full((S,), n, dtype=torch.int32, device=dev)
+    cu = torch.arange(0, (S + 1) * n, n, dtype=torch.int32, device=dev)
+    wide = torch.zeros(S * n, Hq, 132, dtype=torch.bfloat16, device=dev)
+    plain = torch.zeros(S * n, Hq, 128, dtype=torch.bfloat16, device=dev)
+    q = wide[..., 1:129] if variant == "unaligned_q" else plain
+    out = wide[..., 2:130] if variant == "unaligned_out" else torch.empty_like(plain)
+    cb = _cb(3).to(dev)
+    need = _lib.lib().tq_prefill_workspace_bytes(S, n, Hq, Hkv, bt.shape[1], bs)
+    assert need > 32 << 20
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated(dev)
+    torch.cuda.reset_peak_memory_stats(dev)
+    prefill_paged(q, cu, kc, kf, cb, vc, vf, cb, bt, lens, sm_scale=0.0 if variant == "zero_scale" else SM,
+                  q_proj=plain if variant == "q_proj" else None, max_q_len=n, out=out)
+    peak = torch.cuda.max_memory_allocated(dev) - before
+    assert peak >= need if variant == "streams" else peak < 1 << 20

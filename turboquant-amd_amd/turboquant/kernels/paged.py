@@ -654,6 +654,17 @@ PREFILL_CAUSAL = 1
 PREFILL_ROTATE = 2
 
 
+def _prefill_streams(q, out, q_proj, k_fmt: PagedKVFormat, v_fmt: PagedKVFormat, sm_scale: float) -> bool:
+    """Whether tq_prefill_split takes the kernel that uses a workspace (up to 102 MB): lane-grouped tiles, the
+    queries as the QJL operand, a positive scale, query and output rows of whole aligned groups of 8."""
+    if k_fmt.layout != "keys" or v_fmt.layout != "values" or (q_proj is not None and k_fmt.qjl) or not sm_scale > 1e-30:
+        return False
+    for t in (q, out):
+        if (t.stride(0) | t.stride(1)) % 8 or t.data_ptr() % (8 * t.element_size()):
+            return False
+    return True
+
+
 def prefill_paged(
     q: torch.Tensor,
     cu_seqlens_q: torch.Tensor,
@@ -727,9 +738,12 @@ def prefill_paged(
     vv = paged_view(v_cache, v_fmt, vc)
     flags = (PREFILL_CAUSAL if causal else 0) | (PREFILL_ROTATE if rotate else 0)
     mq = T if max_q_len is None else int(max_q_len)
+    scale = float((1.0 / math.sqrt(128)) if sm_scale is None else sm_scale)
     L = _lib.lib()
     # (a buffer of this call: of the current stream, and of the graph under capture)
-    nws = L.tq_prefill_workspace_bytes(S, mq, Hq, Hkv, block_tables.shape[1], k_fmt.block_size)
+    nws = 0
+    if _prefill_streams(q, out, q_proj, k_fmt, v_fmt, scale):
+        nws = L.tq_prefill_workspace_bytes(S, mq, Hq, Hkv, block_tables.shape[1], k_fmt.block_size)
     try:
         ws = torch.empty(nws, dtype=torch.uint8, device=dev) if nws else None
     except torch.OutOfMemoryError:
@@ -740,8 +754,7 @@ def prefill_paged(
         cu_seqlens_q.data_ptr(), S, mq, Hq, Hkv, 128,
         ctypes.byref(kv), ctypes.byref(vv), k_fmt.block_size, k_cache.shape[0],
         block_tables.data_ptr(), block_tables.stride(0), block_tables.shape[1], seq_lens.data_ptr(),
-        float((1.0 / math.sqrt(128)) if sm_scale is None else sm_scale),
-        float((math.sqrt(math.pi / 2) / 128) if corr_scale is None else corr_scale), flags,
+        scale, float((math.sqrt(math.pi / 2) / 128) if corr_scale is None else corr_scale), flags,
         _lib.ptr(ws), nws, out.data_ptr(), _lib.dtype_code(out), out.stride(0), out.stride(1), _lib.stream_handle(dev),
     )
     _lib.check(rc, "tq_prefill_split")
