@@ -319,10 +319,10 @@ void prefill_stream_kernel(TqPrefillStream p) {
     const Share share = share_of(p, P);
     const int nwg = (int)gridDim.x;
     const int wg = (nwg & 7) ? (int)blockIdx.x : (int)((blockIdx.x & 7) * (nwg >> 3) + (blockIdx.x >> 3));
-    const int per = (int)((share.R + nwg - 1) / (uint32_t)nwg);
-    if ((uint32_t)(wg * per) >= share.R) return;  // workgroup-uniform
-    const int w = wg * per + wave;
-    const bool active = wave < per && (uint32_t)w < share.R;
+    const int w0 = (int)(share.R * (uint32_t)wg / (uint32_t)nwg), w1 = (int)(share.R * (uint32_t)(wg + 1) / (uint32_t)nwg);
+    if (w0 == w1) return;  // workgroup-uniform
+    const int w = w0 + wave;
+    const bool active = w < w1;  // (at most kWaves: R <= kWaves nwg)
 
     // ---- tables ----
     {
