@@ -288,3 +288,31 @@ def test_prefill_takes_a_workspace_only_where_it_is_used(dev, variant):
                   q_proj=plain if variant == "q_proj" else None, max_q_len=n, out=out)
     peak = torch.cuda.max_memory_allocated(dev) - before
     assert peak >= need if variant == "streams" else peak < 1 << 20
+
+
+@pytest.mark.parametrize("workspace", [True, False])
+@pytest.mark.parametrize("S", [2, 40])
+@pytest.mark.parametrize("table", [192, 208, 256, 272, 384, 400, 784])
+def test_prefill_dispatch_edges(dev, monkeypatch, table, S, workspace):
+    """Both sides of each line of the dispatch on the block table's tokens, with few and with many segments,
+    with and without a workspace: short sequences in a table of that width, against prefill_kernel (which
+    a separate q_proj selects; both are within RTOL / ATOL of the oracle).  A NaN query row stays NaN."""
+    from turboquant import _lib
+    kb, kq, vb, G, Hkv, bs = 3, True, 3, 6, 4, 16
+    rng = np.random.default_rng(table + S)
+    top = min(table, 300)
+    lens = [top, 0] + [int(x) for x in rng.integers(1, top + 1, S - 2)]
+    n_new = [min(70, n) for n in lens]
+    case = build_case(table, S, G * Hkv, Hkv, lens, kb, kq, vb, bs)
+    wide = np.full((S, table // bs), -1, np.int32)
+    wide[:, :case["bt"].shape[1]] = case["bt"]
+    case["bt"] = wide
+    q, cu = make_queries(rng, n_new, G * Hkv)
+    q[3, 1] = np.nan
+    want, _, _ = run_prefill(dev, case, q, cu, kb, kq, vb, bs, SM, CS, qp=q, out_dtype=torch.float32, max_q_len=70)
+    if not workspace:
+        monkeypatch.setattr(_lib.lib(), "tq_prefill_workspace_bytes", lambda *a: 0)
+    got, _, _ = run_prefill(dev, case, q, cu, kb, kq, vb, bs, SM, CS, out_dtype=torch.float32, max_q_len=70)
+    assert np.isnan(got[3, 1]).all() and np.isnan(want[3, 1]).all()
+    got[3, 1] = want[3, 1] = 0
+    np.testing.assert_allclose(got, want, rtol=2 * RTOL, atol=2 * ATOL)

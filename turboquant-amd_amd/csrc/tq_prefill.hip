@@ -568,11 +568,20 @@ int device_cus(int* cus) {
 // tokens of the stream), and the workspace for their pieces (two per
 // worker) and the cuts' plan.
 constexpr int64_t kStreamWorkers = 256 * kTqPrefillStreamWaves;
-// Block tables of at most this many tokens stay with prefill_kernel: its start is shorter, a workgroup's
-// walk longer (32 query heads on 8 KV heads, 3-bit keys with QJL, no earlier tokens, one / 16 sequences:
-// 32 tokens 18 / 18 us here, 20 / 23 there; 128 tokens 25 / 37 and 27 / 39; 512 tokens after 512 earlier
-// ones 90 / - and 58 / -; one of 640 tokens 62 and 33).
-constexpr int64_t kStreamMinTokens = 192;
+// Calls with block tables of few tokens stay with prefill_kernel, whose start is shorter and whose walk is
+// longer: up to 192 tokens, and with 4-bit keys or values, whose tables take longest to fill, up to 256
+// where its grid leaves it one workgroup per compute unit.  Here / there, 4 bits, 32 / 8 heads: one sequence
+// of 32 tokens 18 / 20 us, of 208 tokens 26.1 / 27.4, four of 256 (256 workgroups) 29.2 / 31.3; sixteen of
+// 208 (896) 57.4 / 45.9; 3 bits, 28 / 4 heads, one of 208 26.3 / 24.8.
+bool stream_long_enough(int64_t prefill_workgroups, bool four_bit, int64_t cap) {
+    return cap > 256 || (cap > 192 && (!four_bit || prefill_workgroups > 256));
+}
+// Tables of at most this many tokens: whole row blocks, no workspace and no merge launch.  A wave's longest
+// row block is no more than what cutting it costs, and the merge (4 to 5 us also where nothing was cut) is
+// left out.  Four sequences of 320 tokens, 4 bits, 32 / 8 heads, here / with a workspace 34.8 / 38.5 us
+// (prefill_kernel 36.7), sixteen of 384 79 / 91; four of 512, 3-bit keys with QJL, 48 / 8 heads 72 / 60
+// with a merge.
+constexpr int64_t kStreamCutTokens = 384;
 int64_t stream_workers(int num_seqs, int max_q_len, int num_q_heads, int num_kv_heads, int64_t cap) {
     const int group = num_q_heads / num_kv_heads;
     const int64_t nrb = ((int64_t)max_q_len * group + kTqPrefillStreamRows - 1) / kTqPrefillStreamRows;
@@ -651,11 +660,13 @@ int prefill_impl(const void* q, int q_dtype, int64_t q_stride_token, int64_t q_s
 
     const int64_t cap = (int64_t)max_blocks_per_seq * block_size;
     const int64_t grid_q = (n_rb * kRowsPerWG + group - 1) / group;  // new tokens that prefill_kernel's grid takes
-    if (cap > kStreamMinTokens && sm_scale > 1e-30f && stream_ok(k, v, q_proj, block_size) && grid_q * group < (1ll << 31) - 64 &&
-        q_vector_ok(q, q_dtype, q_stride_token, q_stride_head) && q_vector_ok(out, out_dtype, out_stride_token, out_stride_head)) {
+    int64_t workers = stream_workers(num_seqs, max_q_len, num_q_heads, num_kv_heads, cap);
+    const bool cut = cap > kStreamCutTokens && workspace && aligned(workspace, 256) && workspace_bytes >= stream_bytes(workers);
+    if (stream_long_enough(grid, k->bits == 4 || v->bits == 4, cap) && sm_scale > 1e-30f && stream_ok(k, v, q_proj, block_size) &&
+        grid_q * group < (1ll << 31) - 64 && q_vector_ok(q, q_dtype, q_stride_token, q_stride_head) &&
+        q_vector_ok(out, out_dtype, out_stride_token, out_stride_head)) {
         int cus = 0;
         if ((rc = device_cus(&cus))) return rc;
-        int64_t workers = stream_workers(num_seqs, max_q_len, num_q_heads, num_kv_heads, cap);
         if (workers > (int64_t)cus * kTqPrefillStreamWaves) workers = (int64_t)cus * kTqPrefillStreamWaves;
         TqPrefillStream t = {};
         t.q = q;
@@ -700,7 +711,7 @@ int prefill_impl(const void* q, int q_dtype, int64_t q_stride_token, int64_t q_s
         t.out_st = out_stride_token;
         t.out_sh = out_stride_head;
         t.n_workers = (int)workers;
-        t.snap = !workspace || !aligned(workspace, 256) || workspace_bytes < stream_bytes(workers);
+        t.snap = !cut;
         if (!t.snap) {
             t.ws_acc = static_cast<float*>(workspace);
             t.ws_ml = t.ws_acc + workers * 2 * kTqPrefillStreamRows * TQ_HEAD_DIM;
@@ -787,7 +798,7 @@ extern "C" size_t tq_prefill_workspace_bytes(int num_seqs, int max_q_len, int nu
         max_blocks_per_seq < 0 || block_size <= 0)
         return 0;
     const int64_t cap = (int64_t)max_blocks_per_seq * block_size;
-    if (cap <= kStreamMinTokens) return 0;
+    if (cap <= kStreamCutTokens) return 0;
     return stream_bytes(stream_workers(num_seqs, max_q_len, num_q_heads, num_kv_heads, cap));
 }
 
