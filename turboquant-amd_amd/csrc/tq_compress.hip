@@ -1206,17 +1206,21 @@ extern "C" int tq_compress_paged_kv(const tq_paged_target* k, const tq_paged_tar
         rc = launch_compress<MODE_PAGED>(pk, k->bits, k->use_qjl, st);
         return rc ? rc : launch_compress<MODE_PAGED>(pv, v->bits, v->use_qjl, st);
     }
-    // K workgroups first, then the V workgroups: of the resident workgroups 29 / 64 take K and the
-    // rest V.  A V wave has the extra pass where runs meet; with halves it was the last to end
-    // (16384 x 8, one run off a multiple of 4: turbo4 28.8 against 20.9 us, turbo3 + QJL 45.0 against
-    // 26.0 us; an aligned run 21.2 against 21.7 us).
+    // K workgroups first, then the V workgroups: half the resident workgroups each, with values in the
+    // values layout 29 / 64 for K.  There the ends of token runs take a second pass and atomics, and they
+    // come at the same place of every head, often a power of two of row groups apart: with halves they all
+    // fall to a few workgroups (16384 x 8, one run off a multiple of 4, 29 / 64 against halves: turbo4
+    // 20.0 / 28.7 us, turbo4 + QJL 26.5 / 45.4; an aligned run 19.7 / 20.2 and 26.4 / 26.3; 31 / 64 is no
+    // better).  Where nothing is gained K's extra round counts: rows layout, 4096 x 8, turbo4 + QJL 10.3
+    // against 8.9 us.
     const int64_t groups = (pk.n_rows + kRowsPerWG - 1) / kRowsPerWG;
+    const bool values = v->tile_layout == TQ_TILE_VALUES;
 #define TQ_KV_DT(B, Q, DT)                                                                          \
     do {                                                                                            \
         static const int res = resident_grid(compress_kv_kernel<B, Q, DT>) / 2;                     \
         const int gk = (int)(groups < res ? groups : (res > 0 ? res : 1));                          \
         hipLaunchKernelGGL((compress_kv_kernel<B, Q, DT>), dim3(2 * gk), dim3(256), 0, st, pk, pv,     \
-                           groups > gk ? gk * 29 / 32 : gk);                                        \
+                           groups > gk && values ? gk * 29 / 32 : gk);                              \
     } while (0)
 #define TQ_KV(B, Q)                                             \
     do {                                                        \
