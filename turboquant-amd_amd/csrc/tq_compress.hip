@@ -785,9 +785,13 @@ __device__ __forceinline__ void compress_rows(const CompressParams& p, int wg, i
 #pragma unroll
                 for (int k = 0; k < 32; ++k) idx[k] = quant_cell(v[k], s_cells);
             } else {
-                float bl[NB];  // read again: this path is rare, and bd would hold its registers through the loop
+                // (this path is rare.  Most instances read the boundaries again, where bd would hold registers
+                // through the loop; unpacked rows without QJL then need 16 more, and fp32 QJL keys wait for it in
+                // each row group: 64 rows of 4 bits 6.1 us, with bd 5.8)
+                constexpr bool kAgain = MODE == MODE_PAGED ? GR || !QJL : QJL;
+                float bl[NB];
 #pragma unroll
-                for (int i = 0; i < NB; ++i) bl[i] = p.boundaries[i];
+                for (int i = 0; i < NB; ++i) bl[i] = kAgain ? p.boundaries[i] : bd[i];
 #pragma unroll
                 for (int k = 0; k < 32; ++k) idx[k] = quant_linear<NB>(v[k], bl);
             }
@@ -918,14 +922,14 @@ __device__ __forceinline__ void compress_any(const CompressParams& p, int wg, in
 // Resident waves per SIMD the paged kernels are compiled for: 4 (128 registers); 3 with QJL keys of 2
 // and 3 bits (the residual row; left to itself the compiler parked 32 registers in AGPRs and ran 2
 // waves: 16384 x 8 turbo3 + QJL / turbo3 25.8 -> 23.1 us, turbo2 + QJL / turbo2 25.2 -> 21.4 us);
-// turbo4 + QJL keeps 2 (3 would spill 12 registers: 25.8 against 26.8 us).
-template <int BITS, int MODE, bool QJL>
+// turbo4 + QJL keeps 2 for 16-bit rows (3 would spill 12 registers: 25.8 against 26.8 us).
+template <int BITS, int MODE, bool QJL, int DT>
 constexpr int compress_min_waves() {
-    return MODE != MODE_PAGED ? 1 : (!QJL ? 4 : (BITS < 4 ? 3 : 1));
+    return MODE != MODE_PAGED ? 1 : (!QJL ? 4 : (BITS < 4 || DT == TQ_F32 ? 3 : 1));
 }
 
 template <int BITS, bool QJL, int MODE, int DT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(compress_min_waves<BITS, MODE, QJL>(), 8)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(compress_min_waves<BITS, MODE, QJL, DT>(), 8)))
 void compress_kernel(CompressParams p) {
     compress_any<BITS, QJL, MODE, DT>(p, blockIdx.x, gridDim.x);
 }
@@ -933,7 +937,7 @@ void compress_kernel(CompressParams p) {
 // K and V of one layer in one launch (same bits; V without QJL): workgroups [0, gk) take K, the
 // rest V.  One launch instead of two halves the fixed cost of a K + V cache update.
 template <int BITS, bool QJL_K, int DT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(compress_min_waves<BITS, MODE_PAGED, QJL_K>(), 8)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(compress_min_waves<BITS, MODE_PAGED, QJL_K, DT>(), 8)))
 void compress_kv_kernel(CompressParams pk, CompressParams pv, int gk) {
     if ((int)blockIdx.x < gk) compress_any<BITS, QJL_K, MODE_PAGED, DT>(pk, blockIdx.x, gk);
     else compress_any<BITS, false, MODE_PAGED, DT>(pv, blockIdx.x - gk, gridDim.x - gk);
