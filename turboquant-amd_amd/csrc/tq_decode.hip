@@ -1011,9 +1011,13 @@ const void* decode_max_kernel_ptr(int kb, bool kq, bool qcols, bool nv) {
 // are fewer than a third of the waves that fit the device; a unit has at least kSplitTiles tiles,
 // about its start-up.  Returns 1 where it stays one pass.  A single pass is a serial chain of ~1.3 us
 // per tile; 24 / 4 heads, turbo3, block 32, one pass against split: 8 x 4096 tokens 341 / 32.6 us,
-// 1 x 16384 1345 / 33.5 us, 1 x 1024 92 / 25 us, 64 x 2048 (8 units each) 181 / 59 us.
+// 1 x 16384 1345 / 33.5 us, 1 x 1024 92 / 25 us, 64 x 2048 (8 units each) 181 / 59 us.  The chain of both
+// passes has to be kSplitGain pairs shorter than one pass, which pays for the second launch and the merge
+// (one pass / split: 100 x 200 tokens, 7 pairs against 2 x 3, 26.9 / 32.9 us; 128 x 256, 8 against 2 x 2,
+// 32.7 / 30.2; 160 x 400, 13 against 2 x 5, 45.5 / 43.4 and with blocks of 16 40.4 / 41.1).
 constexpr int kSplitWaves = 256 * 4 * 2;  // CUs x SIMDs x 2
 constexpr int kSplitTiles = 4;
+constexpr int kSplitGain = 4;
 int single_pass_split(int num_seqs, int num_kv_heads, int limit, int* chunk) {
     const int64_t units = (int64_t)num_seqs * num_kv_heads;
     const int64_t pairs = ((int64_t)limit + 31) / 32;
@@ -1021,6 +1025,7 @@ int single_pass_split(int num_seqs, int num_kv_heads, int limit, int* chunk) {
     n = n < pairs * 2 / kSplitTiles ? n : pairs * 2 / kSplitTiles;
     if (n < 3) return 1;
     const int64_t per = (pairs + n - 1) / n;
+    if (pairs - 2 * per < kSplitGain) return 1;
     *chunk = (int)(32 * per);
     return (int)((pairs + per - 1) / per);
 }
