@@ -534,7 +534,9 @@ def run_decode(
             # room for a split single pass (a caller's own workspace decides that by its size)
             need = L.tq_decode_sparse_workspace_bytes(S, Hq, num_kv_heads, max_seq_len, tokens_per_chunk)
         # (the stream's buffer may be larger: what the call does depends on the call alone)
-        workspace = decode_workspace(dev, need)[:need]
+        workspace, ws_bytes = decode_workspace(dev, need), need
+    else:
+        ws_bytes = workspace.numel()
     if skip_stats is not None and (skip_stats.dtype != torch.int64 or skip_stats.numel() < 2 or not skip_stats.is_cuda):
         raise ValueError("skip_stats must be a device int64 tensor with 2 elements")
     bt_ptr = block_tables.data_ptr() if block_tables is not None else None
@@ -550,7 +552,7 @@ def run_decode(
         _lib.ptr(seq_lens), max_seq_len,
         float(sm_scale), float(corr_scale), float(sparse_threshold),
         tokens_per_chunk,
-        workspace.data_ptr(), workspace.numel(),
+        workspace.data_ptr(), ws_bytes,
         out.data_ptr(), _lib.dtype_code(out), out.stride(0), out.stride(1),
         _lib.ptr(skip_stats),
         _lib.stream_handle(dev),
@@ -660,7 +662,8 @@ def _prefill_streams(q, out, q_proj, k_fmt: PagedKVFormat, v_fmt: PagedKVFormat,
     if k_fmt.layout != "keys" or v_fmt.layout != "values" or (q_proj is not None and k_fmt.qjl) or not sm_scale > 1e-30:
         return False
     for t in (q, out):
-        if (t.stride(0) | t.stride(1)) % 8 or t.data_ptr() % (8 * t.element_size()):
+        st, sh, _ = t.stride()
+        if (st | sh) % 8 or t.data_ptr() % (8 * t.element_size()):
             return False
     return True
 
