@@ -665,246 +665,246 @@ __device__ __forceinline__ void compress_rows(const CompressParams& p, int wg, i
     if constexpr (GR) hf = hadamard_frags<DT>(lane);
 
     for (int64_t row0 = (int64_t)wg * kRowsPerWG; row0 < p.n_rows; row0 += step) {
-      uint64_t link = 0;
-      int first = 0, last = 16;  // the wave's rows, from its base
-      if (VALUES) {
-          int64_t wtok;
-          int whead;
-          const bool wok = locate(row0 + wave16 + (lane - 1), wtok, whead);
-          // (the lane before: wave_shr 1; lane 0's link is not used)
-          const uint32_t plo = __builtin_amdgcn_update_dpp(0, slo, 0x138, 0xf, 0xf, false);
-          bool next_slot = slo == plo + 1;
-          if (p.slot_i64) {
-              const uint32_t phi = __builtin_amdgcn_update_dpp(0, shi, 0x138, 0xf, 0xf, false);
-              next_slot = (((uint64_t)shi << 32) | slo) == (((uint64_t)phi << 32) | plo) + 1;
-          }
-          link = __builtin_amdgcn_ballot_w64(wok && wtok > 0 && next_slot && (slo & 3) != 0);
-          first = __builtin_ctzll(~(link >> 1));
-          last = 16 + __builtin_ctzll(~(link >> 17));
-          s_slots[threadIdx.x & (VALUES ? 255 : 0)] = make_uint2(slo, shi);
-          __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-      }
-      for (int next; first < last; first = next) {
-        // a pass ends at a chunk: rows at its end that go on past 16 are left to the next one
-        next = first + 16;
-        if (VALUES && next < last) {
-            const int b = (int)(link >> (first + 15)) & 7;  // rows first + 14 .. first + 16 continue
-            next -= b == 7 ? 3 : (b >= 6 ? 2 : (b >= 4 ? 1 : 0));
+        uint64_t link = 0;
+        int first = 0, last = 16;  // the wave's rows, from its base
+        if (VALUES) {
+            int64_t wtok;
+            int whead;
+            const bool wok = locate(row0 + wave16 + (lane - 1), wtok, whead);
+            // (the lane before: wave_shr 1; lane 0's link is not used)
+            const uint32_t plo = __builtin_amdgcn_update_dpp(0, slo, 0x138, 0xf, 0xf, false);
+            bool next_slot = slo == plo + 1;
+            if (p.slot_i64) {
+                const uint32_t phi = __builtin_amdgcn_update_dpp(0, shi, 0x138, 0xf, 0xf, false);
+                next_slot = (((uint64_t)shi << 32) | slo) == (((uint64_t)phi << 32) | plo) + 1;
+            }
+            link = __builtin_amdgcn_ballot_w64(wok && wtok > 0 && next_slot && (slo & 3) != 0);
+            first = __builtin_ctzll(~(link >> 1));
+            last = 16 + __builtin_ctzll(~(link >> 17));
+            s_slots[threadIdx.x & (VALUES ? 255 : 0)] = make_uint2(slo, shi);
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            __builtin_amdgcn_wave_barrier();
         }
-        const int end = next < last ? next : last;
-        const int64_t row = row0 + row_in_wg;  // MODE_UNPACKED
-        bool row_ok;
-        int64_t tok;
-        int head;
-        if (MODE == MODE_PAGED) {
-            row_ok = locate(row0 + wave16 + (first + (row_in_wg & 15)), tok, head) && (!VALUES || first + (row_in_wg & 15) < end);
-        } else {
-            row_ok = row < p.n_rows;
-            head = 0;
-            tok = row_ok ? row : 0;
-        }
+        for (int next; first < last; first = next) {
+            // a pass ends at a chunk: rows at its end that go on past 16 are left to the next one
+            next = first + 16;
+            if (VALUES && next < last) {
+                const int b = (int)(link >> (first + 15)) & 7;  // rows first + 14 .. first + 16 continue
+                next -= b == 7 ? 3 : (b >= 6 ? 2 : (b >= 4 ? 1 : 0));
+            }
+            const int end = next < last ? next : last;
+            const int64_t row = row0 + row_in_wg;  // MODE_UNPACKED
+            bool row_ok;
+            int64_t tok;
+            int head;
+            if (MODE == MODE_PAGED) {
+                row_ok = locate(row0 + wave16 + (first + (row_in_wg & 15)), tok, head) && (!VALUES || first + (row_in_wg & 15) < end);
+            } else {
+                row_ok = row < p.n_rows;
+                head = 0;
+                tok = row_ok ? row : 0;
+            }
 
-        // Rows that are not written (padding, past the end) read token 0 of head 0, a row of the
-        // same launch, and their results are dropped: no separate zero fill.
-        int64_t off;
-        const uint32_t lane_off = GR ? 8u * q : 32u * q;
-        if (p.idx32) off = (uint32_t)tok * (uint32_t)p.x_stride_token + (uint32_t)head * (uint32_t)p.x_stride_head + lane_off;
-        else off = tok * p.x_stride_token + (int64_t)head * p.x_stride_head + lane_off;
-        RawRow<DT> raw;
-        if constexpr (GR) load_raw_groups<DT>(p.x, off, raw);
-        else load_raw<DT>(p.x, off, raw);
-        // the slot goes out with the row (token 0's for rows that are not written, whose result
-        // is dropped): its round trip overlaps the row's instead of following the quantisation
-        if (MODE == MODE_PAGED) {
-            int wh;
-            if (VALUES) locate(row0 + step + wave16 + (lane - 1), tok, wh);
-            load_slot(tok, slo, shi);
-        }
-        float v[32];
-        float norm, den, rcp;
-        bool fast;
-        if (MODE == MODE_PAGED) {
-            // v = z, y = scale z (the rotation's scale h, or 1 without rotation)
-            if (p.rotate) {
-                if constexpr (GR) rotate_mfma<DT>(raw, hf, v);
-                else if constexpr (DT == TQ_F32) rotate_unscaled_f32(raw, q, v);
+            // Rows that are not written (padding, past the end) read token 0 of head 0, a row of the
+            // same launch, and their results are dropped: no separate zero fill.
+            int64_t off;
+            const uint32_t lane_off = GR ? 8u * q : 32u * q;
+            if (p.idx32) off = (uint32_t)tok * (uint32_t)p.x_stride_token + (uint32_t)head * (uint32_t)p.x_stride_head + lane_off;
+            else off = tok * p.x_stride_token + (int64_t)head * p.x_stride_head + lane_off;
+            RawRow<DT> raw;
+            if constexpr (GR) load_raw_groups<DT>(p.x, off, raw);
+            else load_raw<DT>(p.x, off, raw);
+            // the slot goes out with the row (token 0's for rows that are not written, whose result
+            // is dropped): its round trip overlaps the row's instead of following the quantisation
+            if (MODE == MODE_PAGED) {
+                int wh;
+                if (VALUES) locate(row0 + step + wave16 + (lane - 1), tok, wh);
+                load_slot(tok, slo, shi);
+            }
+            float v[32];
+            float norm, den, rcp;
+            bool fast;
+            if (MODE == MODE_PAGED) {
+                // v = z, y = scale z (the rotation's scale h, or 1 without rotation)
+                if (p.rotate) {
+                    if constexpr (GR) rotate_mfma<DT>(raw, hf, v);
+                    else if constexpr (DT == TQ_F32) rotate_unscaled_f32(raw, q, v);
+                } else {
+                    raw_to_float<DT>(raw, v);
+                }
+                const float scale = p.rotate ? p.wht_scale : 1.f;
+                const float nz = __builtin_sqrtf(row_sumsq_of<GR>(v));
+                fast = cells && !__builtin_amdgcn_ballot_w64(!(nz < __builtin_huge_valf()));
+                if (fast) {
+                    // x_n = y / (|y| + 1e-8) = z / (|z| + 1e-8 / scale): decisions on z and this
+                    // denominator; 128 / den only places the lookup cell, an approximate reciprocal
+                    // does (it moves x by far less than the cells' eps)
+                    norm = nz * scale;
+                    den = nz + den_eps;
+                    rcp = __builtin_amdgcn_rcpf(den);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 32; ++k) v[k] *= scale;
+                    norm = __builtin_sqrtf(row_sumsq_of<GR>(v));
+                    den = norm + 1e-8f;
+                    rcp = 1.0f / den;
+                }
             } else {
                 raw_to_float<DT>(raw, v);
-            }
-            const float scale = p.rotate ? p.wht_scale : 1.f;
-            const float nz = __builtin_sqrtf(row_sumsq_of<GR>(v));
-            fast = cells && !__builtin_amdgcn_ballot_w64(!(nz < __builtin_huge_valf()));
-            if (fast) {
-                // x_n = y / (|y| + 1e-8) = z / (|z| + 1e-8 / scale): decisions on z and this
-                // denominator; 128 / den only places the lookup cell, an approximate reciprocal
-                // does (it moves x by far less than the cells' eps)
-                norm = nz * scale;
-                den = nz + den_eps;
-                rcp = __builtin_amdgcn_rcpf(den);
-            } else {
-#pragma unroll
-                for (int k = 0; k < 32; ++k) v[k] *= scale;
-                norm = __builtin_sqrtf(row_sumsq_of<GR>(v));
+                if (p.rotate) wht_row(v, q, p.wht_scale);
+                norm = __builtin_sqrtf(row_sumsq(v));
                 den = norm + 1e-8f;
                 rcp = 1.0f / den;
+                // |x| <= 1 unless the norm is not finite (then x may be NaN: searchsorted puts it last)
+                fast = cells && !__builtin_amdgcn_ballot_w64(!(norm < __builtin_huge_valf()));
             }
-        } else {
-            raw_to_float<DT>(raw, v);
-            if (p.rotate) wht_row(v, q, p.wht_scale);
-            norm = __builtin_sqrtf(row_sumsq(v));
-            den = norm + 1e-8f;
-            rcp = 1.0f / den;
-            // |x| <= 1 unless the norm is not finite (then x may be NaN: searchsorted puts it last)
-            fast = cells && !__builtin_amdgcn_ballot_w64(!(norm < __builtin_huge_valf()));
-        }
 
-        int idx[32];
-        float rn = 0.f;
-        uint32_t sbits = 0;
-        if (MODE == MODE_PAGED && fast) {
-            // decisions on z itself (x_n = z / den is never formed); with QJL the residual
-            // r = (x_n - c) norm = (z - c den) (norm / den), its sign that of one fma
-            const float rscale = kCellsRnScale * rcp;
+            int idx[32];
+            float rn = 0.f;
+            uint32_t sbits = 0;
+            if (MODE == MODE_PAGED && fast) {
+                // decisions on z itself (x_n = z / den is never formed); with QJL the residual
+                // r = (x_n - c) norm = (z - c den) (norm / den), its sign that of one fma
+                const float rscale = kCellsRnScale * rcp;
 #pragma unroll
-            for (int k = 0; k < 32; ++k) idx[k] = quant_cell_y(v[k], den, rscale, s_cells);
-            if (QJL) {
-                float r[32];
+                for (int k = 0; k < 32; ++k) idx[k] = quant_cell_y(v[k], den, rscale, s_cells);
+                if (QJL) {
+                    float r[32];
 #pragma unroll
-                for (int k = 0; k < 32; ++k) {
-                    r[k] = __builtin_fmaf(-s_cent[idx[k]], den, v[k]);
-                    sbits |= (r[k] >= 0.f ? 1u : 0u) << k;
+                    for (int k = 0; k < 32; ++k) {
+                        r[k] = __builtin_fmaf(-s_cent[idx[k]], den, v[k]);
+                        sbits |= (r[k] >= 0.f ? 1u : 0u) << k;
+                    }
+                    rn = __builtin_sqrtf(row_sumsq_of<GR>(r)) * (norm / den);
+                    if (norm == 0.f) sbits = 0xffffffffu;  // r = (0 - c) 0 = +-0: sign(0) counts as +1
                 }
-                rn = __builtin_sqrtf(row_sumsq_of<GR>(r)) * (norm / den);
-                if (norm == 0.f) sbits = 0xffffffffu;  // r = (0 - c) 0 = +-0: sign(0) counts as +1
-            }
-        } else {
-#pragma unroll
-            for (int k = 0; k < 32; ++k) v[k] = tq_div_rn(v[k], den, rcp);  // x / (norm + 1e-8)
-            if (fast) {
-#pragma unroll
-                for (int k = 0; k < 32; ++k) idx[k] = quant_cell(v[k], s_cells);
             } else {
-                // (this path is rare.  Most instances read the boundaries again, where bd would hold registers
-                // through the loop; unpacked rows without QJL then need 16 more, and fp32 QJL keys wait for it in
-                // each row group: 64 rows of 4 bits 6.1 us, with bd 5.8)
-                constexpr bool kAgain = MODE == MODE_PAGED ? GR || !QJL : QJL;
-                float bl[NB];
 #pragma unroll
-                for (int i = 0; i < NB; ++i) bl[i] = kAgain ? p.boundaries[i] : bd[i];
+                for (int k = 0; k < 32; ++k) v[k] = tq_div_rn(v[k], den, rcp);  // x / (norm + 1e-8)
+                if (fast) {
 #pragma unroll
-                for (int k = 0; k < 32; ++k) idx[k] = quant_linear<NB>(v[k], bl);
-            }
-            if (QJL) {
-                float r[32];
+                    for (int k = 0; k < 32; ++k) idx[k] = quant_cell(v[k], s_cells);
+                } else {
+                    // (this path is rare.  Most instances read the boundaries again, where bd would hold registers
+                    // through the loop; unpacked rows without QJL then need 16 more, and fp32 QJL keys wait for it in
+                    // each row group: 64 rows of 4 bits 6.1 us, with bd 5.8)
+                    constexpr bool kAgain = MODE == MODE_PAGED ? GR || !QJL : QJL;
+                    float bl[NB];
 #pragma unroll
-                for (int k = 0; k < 32; ++k) {
-                    r[k] = (v[k] - s_cent[idx[k]]) * norm;
-                    sbits |= (r[k] >= 0.f ? 1u : 0u) << k;
-                }
-                rn = __builtin_sqrtf(row_sumsq_of<GR>(r));
-            }
-        }
-
-        if (MODE == MODE_UNPACKED) {
-            if (row_ok) {
-                int64_t* ip = p.indices + row * TQ_HEAD_DIM + 32 * q;
-                float* kp = p.k_mse + row * TQ_HEAD_DIM + 32 * q;
+                    for (int i = 0; i < NB; ++i) bl[i] = kAgain ? p.boundaries[i] : bd[i];
 #pragma unroll
-                for (int k = 0; k < 32; ++k) {
-                    ip[k] = idx[k];
-                    kp[k] = s_cent[idx[k]] * norm;
+                    for (int k = 0; k < 32; ++k) idx[k] = quant_linear<NB>(v[k], bl);
                 }
                 if (QJL) {
-                    float* sp = p.signs + row * TQ_HEAD_DIM + 32 * q;
+                    float r[32];
 #pragma unroll
-                    for (int k = 0; k < 32; ++k) sp[k] = ((sbits >> k) & 1u) ? 1.f : -1.f;
+                    for (int k = 0; k < 32; ++k) {
+                        r[k] = (v[k] - s_cent[idx[k]]) * norm;
+                        sbits |= (r[k] >= 0.f ? 1u : 0u) << k;
+                    }
+                    rn = __builtin_sqrtf(row_sumsq_of<GR>(r));
                 }
-                if (q == 0) {
-                    p.norms[row] = norm;
-                    if (QJL) p.rnorm[row] = rn;
-                }
             }
-        } else {
-            uint2 sw = make_uint2(slo, shi);
-            if (VALUES) sw = s_slots[((threadIdx.x & ~63) + first + (row_in_wg & 15) + 1) & (VALUES ? 255 : 0)];
-            const int64_t slot =
-                !row_ok ? -1 : (p.slot_i64 ? (int64_t)(((uint64_t)sw.y << 32) | sw.x) : (int64_t)(int32_t)sw.x);
-            const bool write = row_ok && slot >= 0 && slot < p.num_blocks * p.block_size;
-            int64_t blk, r_in_blk;
-            if (p.idx32) {
-                const uint32_t sl = write ? (uint32_t)slot : 0u, bs = (uint32_t)p.block_size;
-                const uint32_t b = tq_udiv_apply(sl, p.blk_div);
-                blk = b;
-                r_in_blk = sl - b * bs;
-            } else {
-                blk = write ? slot / p.block_size : 0;
-                r_in_blk = write ? slot - blk * p.block_size : 0;
-            }
-            uint8_t* tile = p.cache + blk * p.stride_block + (int64_t)head * p.stride_head;
-            if (VALUES) {
-                // rows lead_row .. lead_row + 3 of the pass are slots 4k..4k+3
-                const int r16 = row_in_wg & 15, pos = (int)(sw.x & 3), lead_row = r16 - pos;
-                const uint32_t plink = (uint32_t)(link >> (first + 1)) & 0x7ffffu;  // bit r: row r continues row r - 1
-                const bool full = write && lead_row >= 0 && lead_row <= 12 && first + lead_row + 3 < end &&
-                                  ((plink >> ((lead_row + 1) & 31)) & 7) == 7;
-                const uint64_t leaders = __builtin_amdgcn_ballot_w64(full && pos == 0 && q == 0);
-                const int gi = __builtin_popcountll(leaders & ((1ull << ((GR ? lead_row : 4 * lead_row) & 63)) - 1));
-                if (BITS >= 2)
-                    store_values<BITS < 2 ? 2 : BITS, GR>(value_slices<BITS < 2 ? 2 : BITS>(idx), write, full, gi, r16, end - first,
-                                                          plink, tile, r_in_blk, q, s_xchg);
-                if (write && q == 0)
-                    *reinterpret_cast<uint16_t*>(tile + p.off_norm + r_in_blk * p.rs_norm) = (uint16_t)tq_f32_to_f16_bits(norm);
-                continue;
-            }
-            // this lane's 32 indices: 4 * BITS bytes of the row's little-endian bit stream
-            uint32_t w[BITS];
-            if constexpr (GR) {
-                pack_stream_groups<BITS>(idx, w);
-                if (QJL) sbits = sign_bits_groups(sbits);
-            } else {
-                pack_stream<BITS>(idx, w);
-            }
-            if (write) {
-                if (p.tile_layout == TQ_TILE_KEYS) {
-                    // chunk (4n + q) of the row's 16-row sub-tile: index bytes, then sign bytes
-                    constexpr int P = 16 * BITS + (QJL ? 16 : 0), C = 4 * BITS + (QJL ? 4 : 0);
-                    uint32_t* ch = reinterpret_cast<uint32_t*>(tile + (r_in_blk & ~(int64_t)15) * P +
-                                                               (4 * (r_in_blk & 15) + q) * C);
+
+            if (MODE == MODE_UNPACKED) {
+                if (row_ok) {
+                    int64_t* ip = p.indices + row * TQ_HEAD_DIM + 32 * q;
+                    float* kp = p.k_mse + row * TQ_HEAD_DIM + 32 * q;
 #pragma unroll
-                    for (int j = 0; j < BITS; ++j) ch[j] = w[j];
-                    if (QJL) ch[BITS] = sbits;
-                } else {
-                    // row-major regions (this library's rows layout, or caller-described regions
-                    // such as the reference's array-of-slots cache)
-                    uint8_t* ip = tile + r_in_blk * p.rs_idx + 4 * BITS * q;
-                    uint8_t* sp = tile + p.off_signs + r_in_blk * p.rs_sig + 4 * q;
-                    if (!p.narrow) {
+                    for (int k = 0; k < 32; ++k) {
+                        ip[k] = idx[k];
+                        kp[k] = s_cent[idx[k]] * norm;
+                    }
+                    if (QJL) {
+                        float* sp = p.signs + row * TQ_HEAD_DIM + 32 * q;
 #pragma unroll
-                        for (int j = 0; j < BITS; ++j) reinterpret_cast<uint32_t*>(ip)[j] = w[j];
-                        if (QJL) *reinterpret_cast<uint32_t*>(sp) = sbits;
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < BITS; ++j) {
-                            reinterpret_cast<uint16_t*>(ip)[2 * j] = (uint16_t)w[j];
-                            reinterpret_cast<uint16_t*>(ip)[2 * j + 1] = (uint16_t)(w[j] >> 16);
-                        }
-                        if (QJL) {
-                            reinterpret_cast<uint16_t*>(sp)[0] = (uint16_t)sbits;
-                            reinterpret_cast<uint16_t*>(sp)[1] = (uint16_t)(sbits >> 16);
-                        }
+                        for (int k = 0; k < 32; ++k) sp[k] = ((sbits >> k) & 1u) ? 1.f : -1.f;
+                    }
+                    if (q == 0) {
+                        p.norms[row] = norm;
+                        if (QJL) p.rnorm[row] = rn;
                     }
                 }
-                if (q == 0) {
-                    *reinterpret_cast<uint16_t*>(tile + p.off_norm + r_in_blk * p.rs_norm) =
-                        (uint16_t)tq_f32_to_f16_bits(norm);
-                    if (QJL)
-                        *reinterpret_cast<uint16_t*>(tile + p.off_rnorm + r_in_blk * p.rs_norm) =
-                            (uint16_t)tq_f32_to_f16_bits(rn);
+            } else {
+                uint2 sw = make_uint2(slo, shi);
+                if (VALUES) sw = s_slots[((threadIdx.x & ~63) + first + (row_in_wg & 15) + 1) & (VALUES ? 255 : 0)];
+                const int64_t slot =
+                    !row_ok ? -1 : (p.slot_i64 ? (int64_t)(((uint64_t)sw.y << 32) | sw.x) : (int64_t)(int32_t)sw.x);
+                const bool write = row_ok && slot >= 0 && slot < p.num_blocks * p.block_size;
+                int64_t blk, r_in_blk;
+                if (p.idx32) {
+                    const uint32_t sl = write ? (uint32_t)slot : 0u, bs = (uint32_t)p.block_size;
+                    const uint32_t b = tq_udiv_apply(sl, p.blk_div);
+                    blk = b;
+                    r_in_blk = sl - b * bs;
+                } else {
+                    blk = write ? slot / p.block_size : 0;
+                    r_in_blk = write ? slot - blk * p.block_size : 0;
+                }
+                uint8_t* tile = p.cache + blk * p.stride_block + (int64_t)head * p.stride_head;
+                if (VALUES) {
+                    // rows lead_row .. lead_row + 3 of the pass are slots 4k..4k+3
+                    const int r16 = row_in_wg & 15, pos = (int)(sw.x & 3), lead_row = r16 - pos;
+                    const uint32_t plink = (uint32_t)(link >> (first + 1)) & 0x7ffffu;  // bit r: row r continues row r - 1
+                    const bool full = write && lead_row >= 0 && lead_row <= 12 && first + lead_row + 3 < end &&
+                                      ((plink >> ((lead_row + 1) & 31)) & 7) == 7;
+                    const uint64_t leaders = __builtin_amdgcn_ballot_w64(full && pos == 0 && q == 0);
+                    const int gi = __builtin_popcountll(leaders & ((1ull << ((GR ? lead_row : 4 * lead_row) & 63)) - 1));
+                    if (BITS >= 2)
+                        store_values<BITS < 2 ? 2 : BITS, GR>(value_slices<BITS < 2 ? 2 : BITS>(idx), write, full, gi, r16, end - first,
+                                                              plink, tile, r_in_blk, q, s_xchg);
+                    if (write && q == 0)
+                        *reinterpret_cast<uint16_t*>(tile + p.off_norm + r_in_blk * p.rs_norm) = (uint16_t)tq_f32_to_f16_bits(norm);
+                    continue;
+                }
+                // this lane's 32 indices: 4 * BITS bytes of the row's little-endian bit stream
+                uint32_t w[BITS];
+                if constexpr (GR) {
+                    pack_stream_groups<BITS>(idx, w);
+                    if (QJL) sbits = sign_bits_groups(sbits);
+                } else {
+                    pack_stream<BITS>(idx, w);
+                }
+                if (write) {
+                    if (p.tile_layout == TQ_TILE_KEYS) {
+                        // chunk (4n + q) of the row's 16-row sub-tile: index bytes, then sign bytes
+                        constexpr int P = 16 * BITS + (QJL ? 16 : 0), C = 4 * BITS + (QJL ? 4 : 0);
+                        uint32_t* ch = reinterpret_cast<uint32_t*>(tile + (r_in_blk & ~(int64_t)15) * P +
+                                                                   (4 * (r_in_blk & 15) + q) * C);
+#pragma unroll
+                        for (int j = 0; j < BITS; ++j) ch[j] = w[j];
+                        if (QJL) ch[BITS] = sbits;
+                    } else {
+                        // row-major regions (this library's rows layout, or caller-described regions
+                        // such as the reference's array-of-slots cache)
+                        uint8_t* ip = tile + r_in_blk * p.rs_idx + 4 * BITS * q;
+                        uint8_t* sp = tile + p.off_signs + r_in_blk * p.rs_sig + 4 * q;
+                        if (!p.narrow) {
+#pragma unroll
+                            for (int j = 0; j < BITS; ++j) reinterpret_cast<uint32_t*>(ip)[j] = w[j];
+                            if (QJL) *reinterpret_cast<uint32_t*>(sp) = sbits;
+                        } else {
+#pragma unroll
+                            for (int j = 0; j < BITS; ++j) {
+                                reinterpret_cast<uint16_t*>(ip)[2 * j] = (uint16_t)w[j];
+                                reinterpret_cast<uint16_t*>(ip)[2 * j + 1] = (uint16_t)(w[j] >> 16);
+                            }
+                            if (QJL) {
+                                reinterpret_cast<uint16_t*>(sp)[0] = (uint16_t)sbits;
+                                reinterpret_cast<uint16_t*>(sp)[1] = (uint16_t)(sbits >> 16);
+                            }
+                        }
+                    }
+                    if (q == 0) {
+                        *reinterpret_cast<uint16_t*>(tile + p.off_norm + r_in_blk * p.rs_norm) =
+                            (uint16_t)tq_f32_to_f16_bits(norm);
+                        if (QJL)
+                            *reinterpret_cast<uint16_t*>(tile + p.off_rnorm + r_in_blk * p.rs_norm) =
+                                (uint16_t)tq_f32_to_f16_bits(rn);
+                    }
                 }
             }
         }
-      }
     }
 }
 

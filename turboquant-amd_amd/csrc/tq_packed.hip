@@ -281,197 +281,197 @@ void packed_compress_mfma_kernel(PackedParams p) {
         uint32_t rnorm16[kRT];  // fp16 bits, rounded once from the product
 #pragma unroll kPassUnroll
         for (int pass = 0; pass < (PROJ ? 2 : 1); ++pass) {
-        // ---- pass 0: rot^T = PiT^T x_n^T; pass 1: proj^T = PiST^T resid^T ----
-        // K slices in turn (the operands moved up after each), steps of kCB column blocks (with one row
-        // tile two, so that a step has independent products); the A fragments of the next step are
-        // loaded before this step's products (the barrier keeps the schedule to that one step of
-        // look-ahead).
+            // ---- pass 0: rot^T = PiT^T x_n^T; pass 1: proj^T = PiST^T resid^T ----
+            // K slices in turn (the operands moved up after each), steps of kCB column blocks (with one row
+            // tile two, so that a step has independent products); the A fragments of the next step are
+            // loaded before this step's products (the barrier keeps the schedule to that one step of
+            // look-ahead).
 #pragma unroll
-        for (int rt = 0; rt < kRT; ++rt)
+            for (int rt = 0; rt < kRT; ++rt)
 #pragma unroll
-            for (int cb = 0; cb < 8; ++cb) acc[rt][cb] = tq_floatx4{0.f, 0.f, 0.f, 0.f};
-        {
-            const _Float16* mh = s_m1h + pass * (2 * kD * kStride) + n * kStride + 8 * g;
-            tq_half8 ah[2][kCB], al[2][kCB];
-            auto frag = [&](const _Float16* m, int cb, tq_half8 (&h)[kCB], tq_half8 (&l)[kCB]) {
+                for (int cb = 0; cb < 8; ++cb) acc[rt][cb] = tq_floatx4{0.f, 0.f, 0.f, 0.f};
+            {
+                const _Float16* mh = s_m1h + pass * (2 * kD * kStride) + n * kStride + 8 * g;
+                tq_half8 ah[2][kCB], al[2][kCB];
+                auto frag = [&](const _Float16* m, int cb, tq_half8 (&h)[kCB], tq_half8 (&l)[kCB]) {
 #pragma unroll
-                for (int c = 0; c < kCB; ++c) {
-                    h[c] = *reinterpret_cast<const tq_half8*>(m + 16 * (cb + c) * kStride);
-                    l[c] = *reinterpret_cast<const tq_half8*>(m + 16 * (cb + c) * kStride + kD * kStride);
-                }
-            };
-            frag(mh, 0, ah[0], al[0]);
+                    for (int c = 0; c < kCB; ++c) {
+                        h[c] = *reinterpret_cast<const tq_half8*>(m + 16 * (cb + c) * kStride);
+                        l[c] = *reinterpret_cast<const tq_half8*>(m + 16 * (cb + c) * kStride + kD * kStride);
+                    }
+                };
+                frag(mh, 0, ah[0], al[0]);
 #pragma unroll kSliceUnroll
-            for (int ks = 0; ks < 4; ++ks) {
-                const _Float16* next = mh + (ks < 3 ? 32 : 0);
+                for (int ks = 0; ks < 4; ++ks) {
+                    const _Float16* next = mh + (ks < 3 ? 32 : 0);
 #pragma unroll
-                for (int step = 0; step < 8 / kCB; ++step) {
-                    const int cb = kCB * step;
-                    if (cb + kCB < 8) frag(mh, cb + kCB, ah[(step + 1) & 1], al[(step + 1) & 1]);
-                    else frag(next, 0, ah[(step + 1) & 1], al[(step + 1) & 1]);
-                    // hi hi, hi lo, lo hi of each sum, the sums in turn
+                    for (int step = 0; step < 8 / kCB; ++step) {
+                        const int cb = kCB * step;
+                        if (cb + kCB < 8) frag(mh, cb + kCB, ah[(step + 1) & 1], al[(step + 1) & 1]);
+                        else frag(next, 0, ah[(step + 1) & 1], al[(step + 1) & 1]);
+                        // hi hi, hi lo, lo hi of each sum, the sums in turn
 #pragma unroll
-                    for (int part = 0; part < 3; ++part)
+                        for (int part = 0; part < 3; ++part)
 #pragma unroll
-                        for (int i = 0; i < kRT * kCB; ++i) {
-                            const int rt = i / kCB, c = i % kCB;
-                            acc[rt][cb + c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(part < 2 ? ah[step & 1][c] : al[step & 1][c],
-                                                                                     part == 1 ? bl[rt][0] : bh[rt][0],
-                                                                                     acc[rt][cb + c], 0, 0, 0);
+                            for (int i = 0; i < kRT * kCB; ++i) {
+                                const int rt = i / kCB, c = i % kCB;
+                                acc[rt][cb + c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(part < 2 ? ah[step & 1][c] : al[step & 1][c],
+                                                                                         part == 1 ? bl[rt][0] : bh[rt][0],
+                                                                                         acc[rt][cb + c], 0, 0, 0);
+                            }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    mh = next;
+#pragma unroll
+                    for (int rt = 0; rt < kRT; ++rt)
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) {
+                            bh[rt][k] = bh[rt][k + 1];
+                            bl[rt][k] = bl[rt][k + 1];
                         }
-                    __builtin_amdgcn_sched_barrier(0);
                 }
-                mh = next;
+            }
+
+            if (pass == 0) {
+                // ---- indices (BITS-bit fields of the 4 elements of (rt, cb), word 8 rt + cb) and the
+                // elements near a boundary.  Element e = 32 rt + 4 cb + r of a lane is
+                // rot[row0 + 16 rt + n][16 cb + 4 g + r]. ----
+                uint32_t kf[8 * kRT];
+                uint32_t nearw[kRT];
 #pragma unroll
-                for (int rt = 0; rt < kRT; ++rt)
+                for (int rt = 0; rt < kRT; ++rt) {
+                    nearw[rt] = 0;
 #pragma unroll
-                    for (int k = 0; k < 3; ++k) {
-                        bh[rt][k] = bh[rt][k + 1];
-                        bl[rt][k] = bl[rt][k + 1];
+                    for (int cb = 0; cb < 8; ++cb) {
+                        kf[8 * rt + cb] = 0;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            uint32_t k;
+                            float nr;
+                            quantize(acc[rt][cb][r], k, nr);
+                            kf[8 * rt + cb] |= k << (BITS * r);
+                            // shift the sign bit of nr in at bit 0 (one funnel shift): after the 32
+                            // elements, element 4 cb + r of the tile sits at bit 31 - (4 cb + r)
+                            nearw[rt] = __builtin_amdgcn_alignbit(nearw[rt], __float_as_uint(nr), 31);
+                        }
                     }
-            }
-        }
-
-        if (pass == 0) {
-        // ---- indices (BITS-bit fields of the 4 elements of (rt, cb), word 8 rt + cb) and the
-        // elements near a boundary.  Element e = 32 rt + 4 cb + r of a lane is
-        // rot[row0 + 16 rt + n][16 cb + 4 g + r]. ----
-        uint32_t kf[8 * kRT];
-        uint32_t nearw[kRT];
-#pragma unroll
-        for (int rt = 0; rt < kRT; ++rt) {
-            nearw[rt] = 0;
-#pragma unroll
-            for (int cb = 0; cb < 8; ++cb) {
-                kf[8 * rt + cb] = 0;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    uint32_t k;
-                    float nr;
-                    quantize(acc[rt][cb][r], k, nr);
-                    kf[8 * rt + cb] |= k << (BITS * r);
-                    // shift the sign bit of nr in at bit 0 (one funnel shift): after the 32
-                    // elements, element 4 cb + r of the tile sits at bit 31 - (4 cb + r)
-                    nearw[rt] = __builtin_amdgcn_alignbit(nearw[rt], __float_as_uint(nr), 31);
+                    nearw[rt] = __builtin_bitreverse32(nearw[rt]);  // element e at bit e
+                    if (row0 + 16 * rt + n >= p.n_rows) nearw[rt] = 0;
                 }
-            }
-            nearw[rt] = __builtin_bitreverse32(nearw[rt]);  // element e at bit e
-            if (row0 + 16 * rt + n >= p.n_rows) nearw[rt] = 0;
-        }
-        uint64_t near = nearw[0] | (kRT > 1 ? ((uint64_t)nearw[kRT > 1 ? 1 : 0] << 32) : 0ull);
-        // Exact decisions, one near element at a time (about 1e-5 of them): the whole wave
-        // computes that row's norm and dot product in fp64 (x * (1 / (norm + 1e-8)) @ PiT as the
-        // reference orders it) and the owning lane rewrites the element's index field.  The
-        // residual keeps the fp32 value, which is within the threshold of the boundary.
-        while (true) {
-            const uint64_t lanes = __builtin_amdgcn_ballot_w64(near != 0);
-            if (!lanes) break;
-            const int src = __builtin_ctzll(lanes);
-            const uint32_t mlo = __builtin_amdgcn_readlane((uint32_t)near, src);
-            const uint32_t mhi = __builtin_amdgcn_readlane((uint32_t)(near >> 32), src);
-            const int e = mlo ? __builtin_ctz(mlo) : 32 + __builtin_ctz(mhi);
-            const int64_t xo = (row0 + 16 * (e >> 5) + (src & 15)) * p.x_stride;
-            const int col = 16 * ((e >> 2) & 7) + 4 * (src >> 4) + (e & 3);
-            // every lane: dims lane and lane + 64 of the row
-            const double x0 = (double)tq_load1(p.x, xo + lane, DT);
-            const double x1 = (double)tq_load1(p.x, xo + lane + 64, DT);
-            const double dot = wave_sum_f64(__builtin_fma(x1, (double)p.pit[(lane + 64) * kD + col],
-                                                          x0 * (double)p.pit[lane * kD + col]));
-            const double ss = wave_sum_f64(__builtin_fma(x1, x1, x0 * x0));
-            const double exact = dot * (1.0 / (__builtin_sqrt(ss) + 1e-8));
-            uint32_t k = 0;
+                uint64_t near = nearw[0] | (kRT > 1 ? ((uint64_t)nearw[kRT > 1 ? 1 : 0] << 32) : 0ull);
+                // Exact decisions, one near element at a time (about 1e-5 of them): the whole wave
+                // computes that row's norm and dot product in fp64 (x * (1 / (norm + 1e-8)) @ PiT as the
+                // reference orders it) and the owning lane rewrites the element's index field.  The
+                // residual keeps the fp32 value, which is within the threshold of the boundary.
+                while (true) {
+                    const uint64_t lanes = __builtin_amdgcn_ballot_w64(near != 0);
+                    if (!lanes) break;
+                    const int src = __builtin_ctzll(lanes);
+                    const uint32_t mlo = __builtin_amdgcn_readlane((uint32_t)near, src);
+                    const uint32_t mhi = __builtin_amdgcn_readlane((uint32_t)(near >> 32), src);
+                    const int e = mlo ? __builtin_ctz(mlo) : 32 + __builtin_ctz(mhi);
+                    const int64_t xo = (row0 + 16 * (e >> 5) + (src & 15)) * p.x_stride;
+                    const int col = 16 * ((e >> 2) & 7) + 4 * (src >> 4) + (e & 3);
+                    // every lane: dims lane and lane + 64 of the row
+                    const double x0 = (double)tq_load1(p.x, xo + lane, DT);
+                    const double x1 = (double)tq_load1(p.x, xo + lane + 64, DT);
+                    const double dot = wave_sum_f64(__builtin_fma(x1, (double)p.pit[(lane + 64) * kD + col],
+                                                                  x0 * (double)p.pit[lane * kD + col]));
+                    const double ss = wave_sum_f64(__builtin_fma(x1, x1, x0 * x0));
+                    const double exact = dot * (1.0 / (__builtin_sqrt(ss) + 1e-8));
+                    uint32_t k = 0;
 #pragma unroll
-            for (int b = 0; b < NB; ++b) k += exact >= (double)bd[b] ? 1u : 0u;
-            if (lane == src) {
-                const int sh = BITS * (e & 3);
-                kf[e >> 2] = (kf[e >> 2] & ~(((1u << BITS) - 1u) << sh)) | (k << sh);
-                near &= ~(1ull << e);
-            }
-        }
-
-        // ---- indices, residuals, packing ----
-#pragma unroll
-        for (int rt = 0; rt < kRT; ++rt) {
-            const int64_t row = row0 + 16 * rt + n;
-            float rss = 0.f;
-            uint32_t seg[8][BITS > 2 ? 2 : 1];
-#pragma unroll
-            for (int cb = 0; cb < 8; ++cb) {
-                uint64_t f = 0;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float v = acc[rt][cb][r];
-                    const uint32_t k = (kf[8 * rt + cb] >> (BITS * r)) & ((1u << BITS) - 1u);
-                    f |= (uint64_t)k << (BITS * r);
-                    if (PROJ) {
-                        const float rs = v - s_cent[k];
-                        rss = __builtin_fmaf(rs, rs, rss);
-                        // B operand of the second product: slice cb / 2, position 8g + 4 (cb & 1) + r
-                        const _Float16 h = (_Float16)rs;
-                        bh[rt][cb >> 1][4 * (cb & 1) + r] = h;
-                        bl[rt][cb >> 1][4 * (cb & 1) + r] = (_Float16)(rs - (float)h);
+                    for (int b = 0; b < NB; ++b) k += exact >= (double)bd[b] ? 1u : 0u;
+                    if (lane == src) {
+                        const int sh = BITS * (e & 3);
+                        kf[e >> 2] = (kf[e >> 2] & ~(((1u << BITS) - 1u) << sh)) | (k << sh);
+                        near &= ~(1ull << e);
                     }
                 }
-                // this lane's 4 fields sit at bit 4 g BITS of the column block's 16-field segment
-                f <<= 4 * g * BITS;
-                seg[cb][0] = or_over_groups((uint32_t)f);
-                if (BITS > 2) seg[cb][BITS > 2 ? 1 : 0] = or_over_groups((uint32_t)(f >> 32));
-            }
-            if (PROJ) rnorm16[rt] = tq_f32_to_f16_bits(__builtin_sqrtf(sum_over_groups(rss)) * norm32[rt]);
-            if (row < p.n_rows) {
-                // lane group g stores column blocks 2g and 2g + 1: 4 BITS bytes at byte 4 g BITS
-                uint32_t w[BITS];
-                uint64_t sg64[8];
-#pragma unroll
-                for (int cb = 0; cb < 8; ++cb)
-                    sg64[cb] = BITS > 2 ? ((uint64_t)seg[cb][0] | ((uint64_t)seg[cb][BITS > 2 ? 1 : 0] << 32)) : seg[cb][0];
-                const uint64_t s0 = pick_group(sg64, g, 0);
-                const uint64_t s1 = pick_group(sg64, g, 1);
-                // two 16 BITS-bit segments -> 32 BITS bits
-                if (BITS == 1) {
-                    w[0] = (uint32_t)(s0 & 0xffffu) | ((uint32_t)(s1 & 0xffffu) << 16);
-                } else if (BITS == 2) {
-                    w[0] = (uint32_t)s0;
-                    w[BITS > 1 ? 1 : 0] = (uint32_t)s1;
-                } else if (BITS == 3) {
-                    // 48 + 48 bits
-                    w[0] = (uint32_t)s0;
-                    w[1 % BITS] = (uint32_t)(s0 >> 32) | (uint32_t)(s1 << 16);
-                    w[2 % BITS] = (uint32_t)(s1 >> 16);
-                } else {
-                    w[0] = (uint32_t)s0;
-                    w[1 % BITS] = (uint32_t)(s0 >> 32);
-                    w[2 % BITS] = (uint32_t)s1;
-                    w[3 % BITS] = (uint32_t)(s1 >> 32);
-                }
-                uint32_t* dst = reinterpret_cast<uint32_t*>(p.idx_out + row * (16 * BITS) + 4 * g * BITS);
-#pragma unroll
-                for (int j = 0; j < BITS; ++j) dst[j] = w[j];
-                if (g == 0) p.norm_out[row] = (uint16_t)tq_f32_to_f16_bits(norm32[rt]);
-            }
-        }
 
-        } else {
-            // ---- signs (resid went without its factor norm > 0: same signs) ----
+                // ---- indices, residuals, packing ----
 #pragma unroll
-            for (int rt = 0; rt < kRT; ++rt) {
-                const int64_t row = row0 + 16 * rt + n;
-                const bool zero = norm32[rt] == 0.f;  // resid = 0: every projection is 0 -> bit 1
-                uint32_t seg[8];
+                for (int rt = 0; rt < kRT; ++rt) {
+                    const int64_t row = row0 + 16 * rt + n;
+                    float rss = 0.f;
+                    uint32_t seg[8][BITS > 2 ? 2 : 1];
 #pragma unroll
-                for (int cb = 0; cb < 8; ++cb) {
-                    uint32_t f = 0;
+                    for (int cb = 0; cb < 8; ++cb) {
+                        uint64_t f = 0;
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) f |= ((__float_as_uint(acc[rt][cb][r]) >> 31) ^ 1u) << r;
-                    f = zero ? 0xfu : f;
-                    seg[cb] = or_over_groups(f << (4 * g));
+                        for (int r = 0; r < 4; ++r) {
+                            const float v = acc[rt][cb][r];
+                            const uint32_t k = (kf[8 * rt + cb] >> (BITS * r)) & ((1u << BITS) - 1u);
+                            f |= (uint64_t)k << (BITS * r);
+                            if (PROJ) {
+                                const float rs = v - s_cent[k];
+                                rss = __builtin_fmaf(rs, rs, rss);
+                                // B operand of the second product: slice cb / 2, position 8g + 4 (cb & 1) + r
+                                const _Float16 h = (_Float16)rs;
+                                bh[rt][cb >> 1][4 * (cb & 1) + r] = h;
+                                bl[rt][cb >> 1][4 * (cb & 1) + r] = (_Float16)(rs - (float)h);
+                            }
+                        }
+                        // this lane's 4 fields sit at bit 4 g BITS of the column block's 16-field segment
+                        f <<= 4 * g * BITS;
+                        seg[cb][0] = or_over_groups((uint32_t)f);
+                        if (BITS > 2) seg[cb][BITS > 2 ? 1 : 0] = or_over_groups((uint32_t)(f >> 32));
+                    }
+                    if (PROJ) rnorm16[rt] = tq_f32_to_f16_bits(__builtin_sqrtf(sum_over_groups(rss)) * norm32[rt]);
+                    if (row < p.n_rows) {
+                        // lane group g stores column blocks 2g and 2g + 1: 4 BITS bytes at byte 4 g BITS
+                        uint32_t w[BITS];
+                        uint64_t sg64[8];
+#pragma unroll
+                        for (int cb = 0; cb < 8; ++cb)
+                            sg64[cb] = BITS > 2 ? ((uint64_t)seg[cb][0] | ((uint64_t)seg[cb][BITS > 2 ? 1 : 0] << 32)) : seg[cb][0];
+                        const uint64_t s0 = pick_group(sg64, g, 0);
+                        const uint64_t s1 = pick_group(sg64, g, 1);
+                        // two 16 BITS-bit segments -> 32 BITS bits
+                        if (BITS == 1) {
+                            w[0] = (uint32_t)(s0 & 0xffffu) | ((uint32_t)(s1 & 0xffffu) << 16);
+                        } else if (BITS == 2) {
+                            w[0] = (uint32_t)s0;
+                            w[BITS > 1 ? 1 : 0] = (uint32_t)s1;
+                        } else if (BITS == 3) {
+                            // 48 + 48 bits
+                            w[0] = (uint32_t)s0;
+                            w[1 % BITS] = (uint32_t)(s0 >> 32) | (uint32_t)(s1 << 16);
+                            w[2 % BITS] = (uint32_t)(s1 >> 16);
+                        } else {
+                            w[0] = (uint32_t)s0;
+                            w[1 % BITS] = (uint32_t)(s0 >> 32);
+                            w[2 % BITS] = (uint32_t)s1;
+                            w[3 % BITS] = (uint32_t)(s1 >> 32);
+                        }
+                        uint32_t* dst = reinterpret_cast<uint32_t*>(p.idx_out + row * (16 * BITS) + 4 * g * BITS);
+#pragma unroll
+                        for (int j = 0; j < BITS; ++j) dst[j] = w[j];
+                        if (g == 0) p.norm_out[row] = (uint16_t)tq_f32_to_f16_bits(norm32[rt]);
+                    }
                 }
-                if (row < p.n_rows) {
-                    reinterpret_cast<uint32_t*>(p.signs_out + row * 16)[g] = pick_group(seg, g, 0) | (pick_group(seg, g, 1) << 16);
-                    if (g == 0) p.rnorm_out[row] = (uint16_t)rnorm16[rt];
+
+            } else {
+                // ---- signs (resid went without its factor norm > 0: same signs) ----
+#pragma unroll
+                for (int rt = 0; rt < kRT; ++rt) {
+                    const int64_t row = row0 + 16 * rt + n;
+                    const bool zero = norm32[rt] == 0.f;  // resid = 0: every projection is 0 -> bit 1
+                    uint32_t seg[8];
+#pragma unroll
+                    for (int cb = 0; cb < 8; ++cb) {
+                        uint32_t f = 0;
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) f |= ((__float_as_uint(acc[rt][cb][r]) >> 31) ^ 1u) << r;
+                        f = zero ? 0xfu : f;
+                        seg[cb] = or_over_groups(f << (4 * g));
+                    }
+                    if (row < p.n_rows) {
+                        reinterpret_cast<uint32_t*>(p.signs_out + row * 16)[g] = pick_group(seg, g, 0) | (pick_group(seg, g, 1) << 16);
+                        if (g == 0) p.rnorm_out[row] = (uint16_t)rnorm16[rt];
+                    }
                 }
             }
-        }
         }
     }
 }
