@@ -385,8 +385,11 @@ int tq_prefill(const void* q, int q_dtype, int64_t q_stride_token, int64_t q_str
  * tq_prefill with a workspace of tq_prefill_workspace_bytes(...), 256-byte aligned (no initial contents
  * needed; calls that overlap in time must not share one): the key tokens of all row blocks are then
  * shared equally by the device's waves, a row block's keys over several waves where needed, and the
- * pieces merged.  A null or smaller workspace gives tq_prefill.  Same arguments, checks and results
- * otherwise.
+ * pieces merged.  A null or smaller workspace gives tq_prefill.  Same arguments and checks otherwise.
+ * Where a row block is cut depends on the lengths of the whole batch, so a row's result may differ by
+ * fp32 rounding (one step of a 16-bit out_dtype in single elements) between batches, and from tq_prefill;
+ * the same call gives the same bits.  tq_prefill_workspace_bytes is 0 for calls that use none.  Without
+ * one a wave takes whole row blocks: a few new tokens after a long context then run on few waves.
  */
 int tq_prefill_split(const void* q, int q_dtype, int64_t q_stride_token, int64_t q_stride_head,
                      const void* q_proj, int64_t qp_stride_token, int64_t qp_stride_head,

@@ -26,13 +26,20 @@
 // begin there.  A segment inside one worker is written directly; the pieces of a cut one (at most the
 // first and the last of a worker, slots 2w and 2w + 1) go to the workspace and prefill_merge_kernel
 // combines them.  Segments that are no more than the workers and all short are taken whole, one by a
-// worker (16 sequences of 128 tokens: 55 -> 39 us).  Without a workspace (snap) a worker takes the whole
-// segments that begin in its range.
+// worker (16 sequences of 128 tokens: 55 -> 39 us).  Without a workspace, and for short block tables
+// (snap), a worker takes the whole segments that begin in its range.
+// Where a row block is cut follows from all lengths of the call and the number of workers, so a row's
+// fp32 sums are added in an order that depends on the rest of the batch (and on whether there was a
+// workspace): the same row in another batch may differ by fp32 rounding, single outputs by one step of a
+// 16-bit output type.  The same call gives the same bits.
 //
-// Bound: VALU issue and MFMA at two waves per SIMD (256 registers: 96 of accumulators and 48 of q for
-// three row tiles).  48 query heads on 8 KV heads, 4 x 4096 new tokens: 3-bit keys with QJL 2661 ->
-// 1744 us (709 TFLOP/s of products), 4 bits 2207 -> 1444; six sequences of 37..512 new after 1000..16000
-// earlier tokens (32 on 8): 989 -> 152 us, before and after against prefill_kernel.
+// Bound: VALU issue (a step: table addresses, softmax) and MFMA (busy 34 %) at two waves per SIMD (256
+// registers: 96 of accumulators and 48 of q for three row tiles), and the LDS: bank conflicts of the
+// lookups take about a fifth of the time of a compute unit (183 of 860 cycles per step, 3-bit keys with QJL).
+// All instances spill; with QJL keys 7 to 10 values are reloaded in each step, and the wait of a reload
+// behind the next step's key loads also waits for those.  Before / after against prefill_kernel, 48 query
+// heads on 8 KV heads, 4 x 4096 new tokens: 3-bit keys with QJL 2627 -> 1650 us (750 TFLOP/s of products),
+// 4 bits 2207 -> 1350; six sequences of 37..512 new after 1000..16000 earlier tokens (32 on 8): 986 -> 142 us.
 #include "tq_common.h"
 #include "tq_prefill_internal.h"
 
@@ -468,9 +475,8 @@ void prefill_stream_kernel(TqPrefillStream p) {
             constexpr int KW = KB + (KQJL ? 1 : 0);
             uint32_t kw[2][KW], kn[2][2], kr[2][2], vw[2][VB], vn[2][2];
             // The lane's offsets are worked out anew for each step: kept, they are spilled, and a reload waits
-            // for every tile load before it (48 query heads on 8 KV heads, 4 x 4096 tokens: 4-bit 1505 ->
-            // 1432 us, 2-bit with QJL 1810 -> 1640; but 3-bit with QJL, which has other spills, 1720 ->
-            // 1818).
+            // for every tile load before it (48 query heads on 8 KV heads, 4 x 4096 tokens: 4 bits 5 % faster,
+            // 2 bits with QJL 9 %; but 3 bits with QJL, which has other spills, 6 % slower).
             constexpr bool kFresh = !(KB == 3 && KQJL);
             auto load_keys = [&](const Where& o) {
                 const uint32_t l = kFresh ? fresh_lane() : lane, o_k = ((l & 15) * 4 + (l >> 4)) * KC, o_n = 8 * (l >> 4);
@@ -673,7 +679,7 @@ void prefill_stream_kernel(TqPrefillStream p) {
             }
 
             // ---- the piece's rows: acc[a][r] is dim 32g + 8r + a ----
-            const bool whole = j0 == 0 && j1 == nsteps;
+            const bool complete = j0 == 0 && j1 == nsteps;
 #pragma unroll 1
             for (int rt = 0; rt < kRT; ++rt) {
                 const float l = sum_over_groups(lsum[0]);
@@ -682,7 +688,7 @@ void prefill_stream_kernel(TqPrefillStream p) {
                 for (int a = 0; a < 8; ++a)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) o[8 * r + a] = acc[0][a][r];
-                if (whole) {
+                if (complete) {
                     const float inv = l > 0.f ? p.v_cinv / l : 0.f;
 #pragma unroll
                     for (int i = 0; i < 32; ++i) o[i] *= inv;
@@ -776,7 +782,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(TqPrefillStream p) {
                     const int64_t x = (int64_t)(wk == cut.w0 ? cut.slot0 : 2 * wk) * kRows + r0;
                     // (a row without a score to follow, also one whose scores are all NaN: its sums, zero or
                     // NaN, must reach the output.  Here and not where the piece is stored: without the
-                    // select there the loop's registers fall otherwise, 4 x 4096 tokens 1655 -> 1816 us)
+                    // select there the loop's registers fall otherwise, 4 x 4096 tokens 10 % slower)
                     mp[k] = fmaxf(p.ws_ml[2 * x], kNone);
                     lp[k] = p.ws_ml[2 * x + 1];
                     v[k] = *reinterpret_cast<const float4*>(p.ws_acc + x * TQ_HEAD_DIM + 4 * l32);
