@@ -33,12 +33,12 @@
 // workspace): the same row in another batch may differ by fp32 rounding, single outputs by one step of a
 // 16-bit output type.  The same call gives the same bits.
 //
-// Bound: VALU issue (a step: table addresses, softmax) and MFMA (busy 34 %) at two waves per SIMD (256
+// Bound: VALU issue (a step: table addresses, softmax) and MFMA (busy 33 %) at two waves per SIMD (256
 // registers: 96 of accumulators and 48 of q for three row tiles), and the LDS: bank conflicts of the
 // lookups take about a fifth of the time of a compute unit (183 of 860 cycles per step, 3-bit keys with QJL).
-// All instances spill; with QJL keys 7 to 10 values are reloaded in each step, and the wait of a reload
+// All instances spill; with QJL keys 7 to 12 values are reloaded in each step, and the wait of a reload
 // behind the next step's key loads also waits for those.  Before / after against prefill_kernel, 48 query
-// heads on 8 KV heads, 4 x 4096 new tokens: 3-bit keys with QJL 2627 -> 1650 us (750 TFLOP/s of products),
+// heads on 8 KV heads, 4 x 4096 new tokens: 3-bit keys with QJL 2627 -> 1663 us (744 TFLOP/s of products),
 // 4 bits 2207 -> 1350; six sequences of 37..512 new after 1000..16000 earlier tokens (32 on 8): 986 -> 142 us.
 #include "tq_common.h"
 #include "tq_prefill_internal.h"
