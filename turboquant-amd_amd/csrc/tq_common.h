@@ -157,6 +157,19 @@ __device__ __forceinline__ void tq_wht_row_g4(float (&x)[32], float h) {
 #pragma unroll
     for (int i = 0; i < 32; ++i) x[i] = tq_wht_lane(tq_wht_lane(x[i], 16), 32) * h;
 }
+// Max / sum of a value over the four lanes l, l^16, l^32, l^48 (VALU lane swaps, no LDS pipe).
+__device__ __forceinline__ float tq_max_over_groups(float x) {
+    auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    const float y = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(y), __float_as_uint(y), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float tq_sum_over_groups(float x) {
+    auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    const float y = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(y), __float_as_uint(y), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
 // Paged tile geometry (must match tq_tile_bytes / tq_tile_offsets on the host).
 struct tq_tile_geom {
     int64_t off_signs, off_norm, off_rnorm, bytes;

@@ -261,20 +261,6 @@ struct SoftmaxState {
     uint32_t n_skip, n_tot;  // wave-uniform (built from ballots)
 };
 
-// Max / sum of a value over the four lanes l, l^16, l^32, l^48 (VALU lane swaps, no LDS pipe).
-__device__ __forceinline__ float max_over_groups(float x) {
-    auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    const float y = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(y), __float_as_uint(y), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ __forceinline__ float sum_over_groups(float x) {
-    auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    const float y = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(y), __float_as_uint(y), false, false);
-    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
 // Scores of one tile (log2 units; rows at or past nvalid are -inf) and their max over the
 // lane's head column.  kbank: LDS byte address of the lane's bank replica in the K pair table;
 // one = 0x3C003C00 (half2 of 1.0) held in a vector register.
@@ -333,7 +319,7 @@ __device__ __forceinline__ float tile_scores(const TileRaw<KB, KQJL, VB, NV>& cu
         sc[r] = (FULL || 4 * g + r < nvalid) ? v : kNegInf;
         mt = fmaxf(mt, sc[r]);
     }
-    return max_over_groups(mt);
+    return tq_max_over_groups(mt);
 }
 
 // One tile: scores, online softmax, Sparse-V, PV.  FULL: all 16 rows valid (no masking).
@@ -546,7 +532,7 @@ void decode_kernel(DecodeParams p) {
             float amax = 0.f;
 #pragma unroll
             for (int k = 0; k < 32; ++k) amax = fmaxf(amax, fabsf(qpv[k]));
-            amax = max_over_groups(amax);  // lanes (n, g), g = 0..3: the four quarters of head n
+            amax = tq_max_over_groups(amax);  // lanes (n, g), g = 0..3: the four quarters of head n
             if (amax > 0.f && amax < __builtin_huge_valf()) qpe = 12 - ilogbf(amax);
             qpe = qpe < -100 ? -100 : (qpe > 100 ? 100 : qpe);
             qpm = ldexpf(p.qp_scale * p.corr_scale, -qpe);
@@ -681,7 +667,7 @@ void decode_kernel(DecodeParams p) {
         // the running max as the single pass has it here: the maxima of the units before
         const float* pm = p.ws_pm + (s * p.hq + (hvalid ? head : kh * p.group)) * (int64_t)p.n_chunks;
         for (int cb = g; cb < c; cb += 4) sm.m = fmaxf(sm.m, pm[cb]);
-        sm.m = hvalid ? max_over_groups(sm.m) : kNegInf;
+        sm.m = hvalid ? tq_max_over_groups(sm.m) : kNegInf;
     }
     sm.lsum = 0.f;
 #pragma unroll
@@ -769,7 +755,7 @@ void decode_kernel(DecodeParams p) {
                                                          gmask, p, sparse, count, m_blk);
     }
 
-    const float lsum = sum_over_groups(sm.lsum);
+    const float lsum = tq_sum_over_groups(sm.lsum);
     if (count && lane == 0) {
         atomicAdd(p.skip_stats, (unsigned long long)sm.n_skip);
         atomicAdd(p.skip_stats + 1, (unsigned long long)sm.n_tot);

@@ -144,19 +144,6 @@ __device__ __forceinline__ uint32_t wave_incl_scan_u32(uint32_t v) {
     return v;
 }
 
-__device__ __forceinline__ float max_over_groups(float x) {
-    auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    const float y = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(y), __float_as_uint(y), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ __forceinline__ float sum_over_groups(float x) {
-    auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    const float y = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(y), __float_as_uint(y), false, false);
-    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
 // half2 of (vn.lo * p0, vn.hi * p1) for a word vn of two fp16 norms, each product rounded once
 // to nearest: v_fma_mixlo_f16 writes the low half, v_fma_mixhi_f16 the high half keeping the low
 // (two instructions; the compiler forms each half alone and then shifts and ors them).
@@ -314,7 +301,7 @@ __device__ __forceinline__ void compute_pair(const KRaw<KB, KQJL>& kr, const VRa
     // stays within fp16 as with the exact running max, while most pairs skip the rescale of
     // acc and lsum.  The Sparse-V test keeps the exact running max (st.m).
     float mt = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
-    mt = max_over_groups(mt);                 // this tile's max for the lane's head
+    mt = tq_max_over_groups(mt);                 // this tile's max for the lane's head
     const float other = row_swap8f(mt);       // the other tile's max for the same head
     const float m_pair = fmaxf(mt, other);
     const float cexp = p.c_exp;
@@ -968,7 +955,7 @@ void decode_fast_kernel(FastDecodeParams p) {
     }
 
     // ---- combine the lane groups and the two tile halves ----
-    float lsum = sum_over_groups(st.lsum);
+    float lsum = tq_sum_over_groups(st.lsum);
     lsum += row_swap8f(lsum);
     if (SPV == 2) {
         cnt_tot += (unsigned long long)st.n_tot;
@@ -1211,7 +1198,7 @@ void decode_contig_kernel(FastDecodeParams p) {
     }
 
     // ---- combine the lane groups and the two tile halves; acc[a][r] is dim 8(4g + r) + kContigDim[a] ----
-    float lsum = sum_over_groups(st.lsum);
+    float lsum = tq_sum_over_groups(st.lsum);
     lsum += row_swap8f(lsum);
     if (!(c.lo8 && hvalid)) return;
     const float vs = p.v_cinv;

@@ -94,12 +94,6 @@ __device__ __forceinline__ T pick_group(const T (&a)[8], int g, int h) {
     const T x23 = g == 3 ? a[6 + h] : a[4 + h];
     return g >= 2 ? x23 : x01;
 }
-__device__ __forceinline__ float sum_over_groups(float x) {
-    auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    const float y = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(y), __float_as_uint(y), false, false);
-    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
 __device__ __forceinline__ double wave_sum_f64(double x) {
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) x += __shfl_xor(x, o, 64);
@@ -417,7 +411,7 @@ void packed_compress_mfma_kernel(PackedParams p) {
                         seg[cb][0] = or_over_groups((uint32_t)f);
                         if (BITS > 2) seg[cb][BITS > 2 ? 1 : 0] = or_over_groups((uint32_t)(f >> 32));
                     }
-                    if (PROJ) rnorm16[rt] = tq_f32_to_f16_bits(__builtin_sqrtf(sum_over_groups(rss)) * norm32[rt]);
+                    if (PROJ) rnorm16[rt] = tq_f32_to_f16_bits(__builtin_sqrtf(tq_sum_over_groups(rss)) * norm32[rt]);
                     if (row < p.n_rows) {
                         // lane group g stores column blocks 2g and 2g + 1: 4 BITS bytes at byte 4 g BITS
                         uint32_t w[BITS];

@@ -83,19 +83,6 @@ struct PrefillParams {
 
 typedef _Float16 tq_half4v __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ float max_over_groups(float x) {
-    auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    const float y = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(y), __float_as_uint(y), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ __forceinline__ float sum_over_groups(float x) {
-    auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    const float y = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(y), __float_as_uint(y), false, false);
-    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
 // Raw packed data one thread dequantises for a tile.
 struct Raw {
     uint32_t kw[2], vw[2];   // dwords holding the 8 index fields (funnel-shifted by the byte offset)
@@ -455,7 +442,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int rt = 0; rt < kRT; ++rt) {
             float mt = fmaxf(fmaxf(fmaxf(sv[rt][0], sv[rt][1]), fmaxf(sv[rt][2], sv[rt][3])),
                              fmaxf(fmaxf(sv[rt][4], sv[rt][5]), fmaxf(sv[rt][6], sv[rt][7])));
-            mt = max_over_groups(mt);
+            mt = tq_max_over_groups(mt);
             // The exponent base m (per row) moves only when some row's max passes it by more
             // than one log2 unit; p = exp2(s - m - 1) <= 1, and acc and lsum carry the same
             // factor, so most steps skip the rescale.
@@ -503,7 +490,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // ---- normalise, rotate, write ----
 #pragma unroll
     for (int rt = 0; rt < kRT; ++rt) {
-        const float l = sum_over_groups(lsum[rt]);
+        const float l = tq_sum_over_groups(lsum[rt]);
         const float inv = l > 0.f ? p.v_cinv / l : 0.f;
         float o[32];
 #pragma unroll

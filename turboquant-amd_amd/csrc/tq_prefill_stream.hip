@@ -95,19 +95,6 @@ typedef __attribute__((address_space(3))) const uint32_t lds_u32;
 typedef __attribute__((address_space(3))) const tq_u32x2 lds_u32x2;
 typedef __attribute__((address_space(3))) const tq_u32x4 lds_u32x4;
 
-__device__ __forceinline__ float max_over_groups(float x) {
-    auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    const float y = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(y), __float_as_uint(y), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ __forceinline__ float sum_over_groups(float x) {
-    auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    const float y = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(y), __float_as_uint(y), false, false);
-    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
 __device__ __forceinline__ float half_at(const uint32_t* w, int r) {
     const uint32_t b = (r & 1) ? (w[r >> 1] >> 16) : (w[r >> 1] & 0xffffu);
     return (float)__builtin_bit_cast(_Float16, (uint16_t)b);
@@ -649,7 +636,7 @@ void prefill_stream_kernel(TqPrefillStream p) {
                         // M moves only when some row's score passes it, and then kHeadroom above the largest:
                         // p = exp2(c1 s - M) <= 1, and acc and lsum carry the same factor
                         if (__builtin_amdgcn_ballot_w64(__builtin_fmaf(mt, p.c1, -M[rt]) > 0.f)) {
-                            mt = max_over_groups(mt);
+                            mt = tq_max_over_groups(mt);
                             const float Mn = fmaxf(M[rt], __builtin_fmaf(mt, p.c1, kHeadroom));
                             const float alpha = __builtin_amdgcn_exp2f(M[rt] - Mn);
                             lsum[rt] *= alpha;
@@ -682,7 +669,7 @@ void prefill_stream_kernel(TqPrefillStream p) {
             const bool complete = j0 == 0 && j1 == nsteps;
 #pragma unroll 1
             for (int rt = 0; rt < kRT; ++rt) {
-                const float l = sum_over_groups(lsum[0]);
+                const float l = tq_sum_over_groups(lsum[0]);
                 float o[32];
 #pragma unroll
                 for (int a = 0; a < 8; ++a)
