@@ -78,7 +78,7 @@ struct DecodeParams {
     float* ws_m;       // [num_seqs][hq][n_chunks]  (log2 domain)
     float* ws_l;
     float* ws_pm;      // split single pass: [num_seqs][hq][n_chunks] score maxima (log2 domain), or null
-    int len_limit;     // tokens of a sequence that are processed
+    int len_limit;     // tokens of a sequence that are processed (at most the block table's)
     unsigned long long* skip_stats;
     void* out;
     int out_dtype;
@@ -480,8 +480,6 @@ void decode_kernel(DecodeParams p) {
     if (s >= p.num_seqs) return;
 
     int L = tq_seq_len(p.seq_lens, s, p.uniform_len);
-    const int cap = p.max_blocks * p.block_size;
-    L = L < cap ? L : cap;
     L = L < p.len_limit ? L : p.len_limit;
     const int t_begin = c * p.chunk;
     if (t_begin >= L) return;
